@@ -220,6 +220,17 @@ inline unsigned sched_grid(long Vh, int nblk, int block, int xcd, int pinter, in
     return (unsigned)g;
 }
 
+// grid of clgd::tile64_site: 8 tiles of at most ceil(L0 / TX) x ceil(L1 / TY) planes
+inline unsigned tile64_grid(const Geo& g, int nblk, int TY) {
+    const int plane = g.L[2] * g.L[3] / 2, TX = 8 / TY;
+    return 8u * (unsigned)(nblk * ((plane + 63) / 64) * ((g.L[0] + TX - 1) / TX) * ((g.L[1] + TY - 1) / TY));
+}
+// whether that schedule keeps at least 7/8 of its lanes busy
+inline bool tile64_fits(const Geo& g, int TY) {
+    const long lanes = 64L * tile64_grid(g, 1, TY);
+    return 8L * g.Vh >= 7L * lanes;
+}
+
 }  // namespace clg
 
 // ======================================================================= device side
@@ -334,19 +345,24 @@ __device__ __forceinline__ unsigned logical_wg(int xcd) {
     }
     return wg;
 }
-// site (p, h) of this thread in logical block lb of blockDim.x sites
-__device__ __forceinline__ bool block_site(unsigned lb, int Vh, int nblk, int pbase, int pinter, int& p, int& h) {
+// site (p, h) of lane `tid` in logical block lb of `bs` sites
+__device__ __forceinline__ bool block_site(unsigned lb, unsigned bs, unsigned tid, int Vh, int nblk, int pbase, int pinter,
+                                           int& p, int& h) {
     if (nblk == 2 && pinter) {
         p = (int)(lb & 1u);
-        h = (int)((lb >> 1) * blockDim.x + threadIdx.x);
+        h = (int)((lb >> 1) * bs + tid);
         return h < Vh;
     }
-    const long gid = (long)lb * blockDim.x + threadIdx.x;
+    const long gid = (long)lb * bs + tid;
     if (gid >= (long)nblk * Vh) return false;
     const int blk = (int)(gid / Vh);
     h = (int)(gid - (long)blk * Vh);
     p = nblk == 2 ? blk : pbase;
     return true;
+}
+// the same for one site per thread: logical block lb of blockDim.x sites
+__device__ __forceinline__ bool block_site(unsigned lb, int Vh, int nblk, int pbase, int pinter, int& p, int& h) {
+    return block_site(lb, blockDim.x, threadIdx.x, Vh, nblk, pbase, pinter, p, h);
 }
 // Tiled plane schedule for launches of one workgroup per (x,y) plane (blockDim = L2*L3/2 sites of one
 // parity; nblk = 2 interleaves the parities plane by plane): the L0 x L1 grid of planes is cut into
@@ -372,6 +388,32 @@ __device__ __forceinline__ unsigned tile_block(const clg::Geo& g, int nblk, int 
     }
     const unsigned P = (unsigned)((ix * tx + xl) * g.L[1] + iy * ty + yl);
     return nblk == 2 ? 2u * P + par : P;
+}
+// The same schedule in blocks of 64 sites for any lattice: a plane's L2*L3/2 sites of one parity are
+// ceil(plane / 64) blocks (the last one partly idle), the tile borders are rounded where the extents do not
+// divide, and an XCD with a smaller tile leaves its last blocks idle.  Grid: tile64_grid.  What it buys
+// over XCD slabs is the reuse distance in x: at 24^3x48 a slab step is 10.6 MB of FP32 links and spinors,
+// past the 4 MB L2, a tile step 2.6 MB (direction-split FP32 half hop 46 -> 38 us, FP64 D 200 -> 158 us).
+__device__ __forceinline__ bool tile64_site(const clg::Geo& g, int nblk, int pbase, int TY, int ymajor, int lane, int& p,
+                                            int& h) {
+    const int plane = g.L[2] * g.L[3] / 2, nsub = (plane + 63) / 64, TX = 8 / TY;
+    const int k = (int)(blockIdx.x & 7u), j = (int)(blockIdx.x >> 3);
+    const int ix = k / TY, iy = k % TY;
+    const int x0 = ix * g.L[0] / TX, y0 = iy * g.L[1] / TY;
+    const int tx = (ix + 1) * g.L[0] / TX - x0, ty = (iy + 1) * g.L[1] / TY - y0;
+    const int sub = j % nsub;
+    int q = j / nsub;
+    p = pbase;
+    if (nblk == 2) {
+        p = q & 1;
+        q >>= 1;
+    }
+    h = 0;
+    if (q >= tx * ty) return false;
+    const int major = q / (ymajor ? tx : ty), minor = q - major * (ymajor ? tx : ty);
+    const int x = x0 + (ymajor ? minor : major), y = y0 + (ymajor ? major : minor);
+    h = (x * g.L[1] + y) * plane + sub * 64 + lane;
+    return sub * 64 + lane < plane;
 }
 __device__ __forceinline__ bool map_site(int Vh, int nblk, int pbase, int xcd, int pinter, int& p, int& h) {
     return block_site(logical_wg(xcd), Vh, nblk, pbase, pinter, p, h);
@@ -502,6 +544,20 @@ template <> struct WilsonIO<CLG_F64> {
 #pragma unroll
         for (int k = 0; k < 12; ++k) stq<double2, NT>(b, Vh, k, e, make_double2((double)v[k].x, (double)v[k].y));
     }
+    // components 4 w .. 4 w + 3 only (a third of the site)
+    template <typename R>
+    __device__ __forceinline__ static void load4(const char* b, const float*, int Vh, unsigned e, unsigned, int w, C2<R>* v) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const double2 a = ldp<double2>(b, Vh, 4 * w + k, e);
+            v[k] = C2<R>{(R)a.x, (R)a.y};
+        }
+    }
+    template <typename R, bool NT = false>
+    __device__ __forceinline__ static void store4(char* b, int Vh, unsigned e, int w, const C2<R>* v) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) stq<double2, NT>(b, Vh, 4 * w + k, e, make_double2((double)v[k].x, (double)v[k].y));
+    }
 };
 
 template <> struct WilsonIO<CLG_F32> {
@@ -522,6 +578,22 @@ template <> struct WilsonIO<CLG_F32> {
         for (int k = 0; k < 6; ++k)
             stq<float4, NT>(b, Vh, k, e,
                             make_float4((float)v[2 * k].x, (float)v[2 * k].y, (float)v[2 * k + 1].x, (float)v[2 * k + 1].y));
+    }
+    template <typename R>
+    __device__ __forceinline__ static void load4(const char* b, const float*, int Vh, unsigned e, unsigned, int w, C2<R>* v) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const float4 a = ldp<float4>(b, Vh, 2 * w + k, e);
+            v[2 * k] = C2<R>{(R)a.x, (R)a.y};
+            v[2 * k + 1] = C2<R>{(R)a.z, (R)a.w};
+        }
+    }
+    template <typename R, bool NT = false>
+    __device__ __forceinline__ static void store4(char* b, int Vh, unsigned e, int w, const C2<R>* v) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            stq<float4, NT>(b, Vh, 2 * w + k, e,
+                        make_float4((float)v[2 * k].x, (float)v[2 * k].y, (float)v[2 * k + 1].x, (float)v[2 * k + 1].y));
     }
 };
 
@@ -574,6 +646,27 @@ template <> struct WilsonIO<CLG_F16> {
             stq<uint4, NT>(b, Vh, k, e, a);
         }
     }
+    template <typename R>
+    __device__ __forceinline__ static void load4(const char* b, const float* nb, int Vh, unsigned e, unsigned ne, int w,
+                                                 C2<R>* v) {
+        const float s = nb[ne];
+        const uint4 a = ldp<uint4>(b, Vh, w, e);
+        float2 f;
+        f = unpack_h2(a.x); v[0] = C2<R>{(R)(f.x * s), (R)(f.y * s)};
+        f = unpack_h2(a.y); v[1] = C2<R>{(R)(f.x * s), (R)(f.y * s)};
+        f = unpack_h2(a.z); v[2] = C2<R>{(R)(f.x * s), (R)(f.y * s)};
+        f = unpack_h2(a.w); v[3] = C2<R>{(R)(f.x * s), (R)(f.y * s)};
+    }
+    // v already divided by the site scale, which the caller stores
+    template <typename R, bool NT = false>
+    __device__ __forceinline__ static void store4(char* b, int Vh, unsigned e, int w, const C2<R>* v) {
+        uint4 a;
+        a.x = pack_h2((float)v[0].x, (float)v[0].y);
+        a.y = pack_h2((float)v[1].x, (float)v[1].y);
+        a.z = pack_h2((float)v[2].x, (float)v[2].y);
+        a.w = pack_h2((float)v[3].x, (float)v[3].y);
+        stq<uint4, NT>(b, Vh, w, e, a);
+    }
 };
 
 // Staggered vector: 3 complex per site, one complex per plane (16 / 8 / 4 bytes)
@@ -590,6 +683,16 @@ template <> struct KSIO<CLG_F64> {
 #pragma unroll
         for (int k = 0; k < 3; ++k) stp<double2>(b, Vh, k, e, make_double2((double)v[k].x, (double)v[k].y));
     }
+    // colour k only
+    template <typename R>
+    __device__ __forceinline__ static void load1(const char* b, int Vh, int k, unsigned e, C2<R>& v) {
+        const double2 a = ldp<double2>(b, Vh, k, e);
+        v = C2<R>{(R)a.x, (R)a.y};
+    }
+    template <typename R>
+    __device__ __forceinline__ static void store1(char* b, int Vh, int k, unsigned e, C2<R> v) {
+        stp<double2>(b, Vh, k, e, make_double2((double)v.x, (double)v.y));
+    }
 };
 template <> struct KSIO<CLG_F32> {
     static constexpr int NPL = 3;
@@ -602,6 +705,16 @@ template <> struct KSIO<CLG_F32> {
     __device__ __forceinline__ static void store(char* b, float*, int Vh, unsigned e, unsigned, const C2<R>* v) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) stp<float2>(b, Vh, k, e, make_float2((float)v[k].x, (float)v[k].y));
+    }
+    // colour k only
+    template <typename R>
+    __device__ __forceinline__ static void load1(const char* b, int Vh, int k, unsigned e, C2<R>& v) {
+        const float2 a = ldp<float2>(b, Vh, k, e);
+        v = C2<R>{(R)a.x, (R)a.y};
+    }
+    template <typename R>
+    __device__ __forceinline__ static void store1(char* b, int Vh, int k, unsigned e, C2<R> v) {
+        stp<float2>(b, Vh, k, e, make_float2((float)v.x, (float)v.y));
     }
 };
 template <> struct KSIO<CLG_F16> {

@@ -39,6 +39,7 @@ struct KSArgs {
     int xcd, pinter;  // work decomposition (clgd::map_site)
     const char* x;    // hop mode 2: out = a H in + two_am * x
     const float* xn;
+    int tile_y, tile_ymaj;  // tiled plane schedule (clgd::tile64_site) when tile_y > 0
     int mode;         // 0: D on full fields; 1: out = a H in; 2: out = a H in + b x (half fields)
 };
 
@@ -132,11 +133,108 @@ __global__ __launch_bounds__(256) void k_ks(KSArgs a) {
     SIO::store(a.out, a.outn, a.g.Vh, eo, no, o);
 }
 
+// ---- direction-split form: a workgroup of 8 waves takes 64 sites, one direction (mu, forward or backward)
+// per wave; each wave leaves its signed, link-multiplied colour vector in LDS, and after one barrier wave
+// c < 3 sums colour c, adds the mass or x term and stores.  Eight times the waves for a small lattice, and
+// both users of a link in one L2 more often on a large one.  Measured (us, one site per thread -> split):
+// FP64 D 21x19x25x18 27.1 -> 24.7, 24^3x24 47.9 -> 36.2 (tiled order), 24^3x48 108 -> 91, FP32 24^3x16
+// 17.4 -> 15.3; FP16 storage loses from 12^3x24 on (5.0 against 5.4).  The tuner times both.
+constexpr int kSplitSites = 64;
+
+template <int MU, bool FWD, typename R, class SIO, class LIO>
+__device__ __forceinline__ void ks_split_dir(const KSArgs& a, const Site& s, int p, int h, C2<R>* t) {
+    C2<R> v[3], u[9];
+    const int Vh = a.g.Vh;
+    const Nbr n = FWD ? fwd_nbr<MU>(a.g, s, p) : bwd_nbr<MU>(a.g, s, p);
+    const unsigned pe = a.in_full ? (unsigned)n.p : 0u;
+    SIO::load(a.in, a.inn, Vh, pe * SIO::NPL * Vh + n.h, pe * Vh + n.h, v);
+    if constexpr (FWD) {
+        LIO::load(a.gauge, Vh, (unsigned)(p * 4 + MU) * LIO::NPL * Vh + h, u);
+        su3_mv(u, v, t);
+    } else {
+        LIO::load(a.gauge, Vh, (unsigned)(n.p * 4 + MU) * LIO::NPL * Vh + n.h, u);
+        su3_mdv(u, v, t);
+    }
+    const int e = eta_sign<MU>(s) * n.sign;
+    if ((FWD ? e : -e) < 0) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) t[c] = cmk<R>(-t[c].x, -t[c].y);
+    }
+}
+
+template <typename R, int SP, int GP, int RECON, int MODE>
+__global__ __launch_bounds__(8 * kSplitSites) void k_ks_split(KSArgs a) {
+    typedef KSIO<SP> SIO;
+    typedef LinkIO<GP, RECON> LIO;
+    constexpr bool SCALED = SP == CLG_F16;
+    constexpr int NC = SCALED ? 3 : 1;  // FP16 storage: one wave needs all three colours for the site scale
+    __shared__ C2<R> sm[8 * 3 * kSplitSites];
+    const int lane = (int)threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int Vh = a.g.Vh;
+    int p, h;
+    const bool valid = a.tile_y > 0 ? tile64_site(a.g, a.nblk, a.pbase, a.tile_y, a.tile_ymaj, lane, p, h)
+                                    : block_site(logical_wg(a.xcd), kSplitSites, (unsigned)lane, Vh, a.nblk, a.pbase,
+                                                 a.pinter, p, h);
+    const unsigned po = a.out_full ? (unsigned)p : 0u;
+    const unsigned eo = po * SIO::NPL * Vh + h, no = po * Vh + h;
+    const bool mine = valid && w < (SCALED ? 1 : 3);
+    C2<R> xv[NC];
+    if (valid) {
+        if constexpr (MODE != 1) {
+            if (mine) {
+                const char* xp = MODE == 0 ? a.in : a.x;
+                const float* xn = MODE == 0 ? a.inn : a.xn;
+                const unsigned pi = (MODE == 0 ? a.in_full : a.out_full) ? (unsigned)p : 0u;
+                if constexpr (SCALED) SIO::load(xp, xn, Vh, pi * SIO::NPL * Vh + h, pi * Vh + h, xv);
+                else SIO::load1(xp, Vh, w, pi * SIO::NPL * Vh + h, xv[0]);
+            }
+        }
+        const Site s = site_of(a.g, p, h);
+        C2<R> t[3];
+        switch (w) {
+            case 0: ks_split_dir<0, true, R, SIO, LIO>(a, s, p, h, t); break;
+            case 1: ks_split_dir<0, false, R, SIO, LIO>(a, s, p, h, t); break;
+            case 2: ks_split_dir<1, true, R, SIO, LIO>(a, s, p, h, t); break;
+            case 3: ks_split_dir<1, false, R, SIO, LIO>(a, s, p, h, t); break;
+            case 4: ks_split_dir<2, true, R, SIO, LIO>(a, s, p, h, t); break;
+            case 5: ks_split_dir<2, false, R, SIO, LIO>(a, s, p, h, t); break;
+            case 6: ks_split_dir<3, true, R, SIO, LIO>(a, s, p, h, t); break;
+            default: ks_split_dir<3, false, R, SIO, LIO>(a, s, p, h, t); break;
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) sm[(w * 3 + c) * kSplitSites + lane] = t[c];
+    }
+    __syncthreads();
+    if (!mine) return;
+    C2<R> o[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        const int c = SCALED ? k : w;
+        C2<R> acc = sm[c * kSplitSites + lane];
+#pragma unroll
+        for (int d = 1; d < 8; ++d) acc = cadd(acc, sm[(d * 3 + c) * kSplitSites + lane]);
+        if constexpr (MODE == 0) {
+            const R m = (R)a.two_am, hs = (R)a.hs;
+            o[k] = cmul(cmk<R>((R)a.cr, (R)a.ci), cmk<R>(m * xv[k].x + hs * acc.x, m * xv[k].y + hs * acc.y));
+        } else {
+            const R ar = (R)a.cr, br = (R)a.two_am;
+            o[k] = cmk<R>(ar * acc.x, ar * acc.y);
+            if constexpr (MODE == 2) { o[k].x += br * xv[k].x; o[k].y += br * xv[k].y; }
+        }
+    }
+    if constexpr (SCALED) SIO::store(a.out, a.outn, Vh, eo, no, o);
+    else SIO::store1(a.out, Vh, w, eo, o[0]);
+}
+
 struct KSCfg {
-    int block;  // threads per workgroup
-    int xcd;    // 0: hardware order; 8: XCD-contiguous slabs, parities interleaved block by block
-    int pm;     // 0 or 2 (ks_mu)
+    int block;  // threads per workgroup (kSplitPm: sites per workgroup, kSplitSites)
+    int xcd;    // 0: hardware order; 8: XCD-contiguous slabs, parities interleaved block by block;
+                // kSplitPm only: 10*TY + m, the tiled plane schedule in 64-site blocks (m = 1: y-major)
+    int pm;     // 0 or 2 (ks_mu); kSplitPm: the direction-split kernel
 };
+constexpr int kSplitPm = 9;
+inline bool ks_tiled(int xcd) { return (xcd / 10 == 2 || xcd / 10 == 4 || xcd / 10 == 8) && xcd % 10 <= 1; }
 
 template <typename R, int SP, int GP, int RECON, int PM>
 void ks_launch_pm(const KSArgs& a0, hipStream_t st, const KSCfg& c) {
@@ -150,8 +248,27 @@ void ks_launch_pm(const KSArgs& a0, hipStream_t st, const KSCfg& c) {
 }
 
 template <typename R, int SP, int GP, int RECON>
+void ks_launch_split(const KSArgs& a0, hipStream_t st, const KSCfg& c) {
+    KSArgs a = a0;
+    unsigned grid;
+    if (ks_tiled(c.xcd)) {
+        a.tile_y = c.xcd / 10;
+        a.tile_ymaj = c.xcd % 10;
+        grid = tile64_grid(a.g, a.nblk, a.tile_y);
+    } else {
+        a.xcd = c.xcd;
+        a.pinter = c.xcd > 1 ? 1 : 0;
+        grid = sched_grid(a.g.Vh, a.nblk, kSplitSites, a.xcd, a.pinter);
+    }
+    if (a.mode == 2) k_ks_split<R, SP, GP, RECON, 2><<<grid, 8 * kSplitSites, 0, st>>>(a);
+    else if (a.mode == 1) k_ks_split<R, SP, GP, RECON, 1><<<grid, 8 * kSplitSites, 0, st>>>(a);
+    else k_ks_split<R, SP, GP, RECON, 0><<<grid, 8 * kSplitSites, 0, st>>>(a);
+}
+
+template <typename R, int SP, int GP, int RECON>
 void ks_launch_t(const KSArgs& a, hipStream_t st, const KSCfg& c) {
-    if (c.pm == 2) ks_launch_pm<R, SP, GP, RECON, 2>(a, st, c);
+    if (c.pm == kSplitPm) ks_launch_split<R, SP, GP, RECON>(a, st, c);
+    else if (c.pm == 2) ks_launch_pm<R, SP, GP, RECON, 2>(a, st, c);
     else ks_launch_pm<R, SP, GP, RECON, 0>(a, st, c);
 }
 
@@ -194,11 +311,18 @@ std::string& ks_loaded() {  // the tuning-cache file whose entries are in ks_tab
 }
 
 bool ks_valid(const KSCfg& c) {
+    if (c.pm == kSplitPm) return c.block == kSplitSites && (c.xcd == 0 || c.xcd == 8 || ks_tiled(c.xcd));
     return (c.block == 64 || c.block == 128 || c.block == 256) && (c.xcd == 0 || c.xcd == 8) && (c.pm == 0 || c.pm == 2);
 }
 
+// Untuned launches (tuning off, small lattices, graph capture) take the direction split up to this many
+// sites: measured, it is level with one site per thread or ahead of it for FP64 and FP32 vectors (FP64 D at
+// 24^3x16 29.2 against 32.5 us) and behind in FP16 from 12^3x24 on (5.4 against 5.0 us).
+inline long split_default_max(int prec) { return prec == CLG_F16 ? 32768 : 262144; }
+
 int ks_launch(const KSArgs& a, int prec, int gprec, bool r12, hipStream_t st) {
-    KSCfg cfg{256, 8, 0};
+    const long nsite = (long)a.nblk * a.g.Vh;
+    KSCfg cfg = nsite <= split_default_max(prec) ? KSCfg{kSplitSites, 8, kSplitPm} : KSCfg{256, 8, 0};
     // CLG_TUNE_FORCE_KS="block,xcd,pin" fixes the launch configuration (testing and profiling)
     if (const char* e = std::getenv("CLG_TUNE_FORCE_KS")) {
         KSCfg f{0, 0, 0};
@@ -238,26 +362,38 @@ int ks_launch(const KSArgs& a, int prec, int gprec, bool r12, hipStream_t st) {
     (void)hipStreamIsCapturing(st, &cs);
     const bool aliased = a.mode == 2 && a.x == a.out;  // repeated candidate launches would compound
     if (need_tune && tuning_enabled() && !aliased && cs == hipStreamCaptureStatusNone && (long)a.nblk * a.g.Vh >= 4096) {
-        const KSCfg cands[] = {{64, 0, 2}, {128, 0, 2}, {256, 0, 2}, {64, 8, 2}, {128, 8, 2}, {256, 8, 2},
-                               {64, 8, 0}, {128, 8, 0}, {256, 8, 0}};
+        std::vector<KSCfg> cands = {{64, 0, 2}, {128, 0, 2}, {256, 0, 2}, {64, 8, 2}, {128, 8, 2}, {256, 8, 2},
+                               {64, 8, 0}, {128, 8, 0}, {256, 8, 0},
+                               {kSplitSites, 0, kSplitPm}, {kSplitSites, 8, kSplitPm}};
         hipEvent_t e0, e1;
         CLG_HIP(hipEventCreate(&e0));
         CLG_HIP(hipEventCreate(&e1));
         float best = 1e30f;
+        for (int TY : {2, 4, 8})
+            if (tile64_fits(a.g, TY))
+                for (int m : {0, 1}) cands.push_back(KSCfg{kSplitSites, 10 * TY + m, kSplitPm});
         for (const KSCfg& c : cands) {
             CLG_TRY(ks_launch_cfg(a, prec, gprec, r12, st, c));  // warm
-            CLG_HIP(hipEventRecord(e0, st));
-            for (int r = 0; r < 3; ++r) CLG_TRY(ks_launch_cfg(a, prec, gprec, r12, st, c));
-            CLG_HIP(hipEventRecord(e1, st));
-            CLG_HIP(hipEventSynchronize(e1));
-            float ms = 0.f;
-            CLG_HIP(hipEventElapsedTime(&ms, e0, e1));
+            float ms = 0.f;  // of three launches
+            // a launch of a few microseconds is timed again over more of them: three are within the clock's noise
+            for (int reps : {3, 15}) {
+                if (reps == 15 && (ms > 0.12f || ms > 1.3f * best)) break;
+                CLG_HIP(hipEventRecord(e0, st));
+                for (int r = 0; r < reps; ++r) CLG_TRY(ks_launch_cfg(a, prec, gprec, r12, st, c));
+                CLG_HIP(hipEventRecord(e1, st));
+                CLG_HIP(hipEventSynchronize(e1));
+                CLG_HIP(hipEventElapsedTime(&ms, e0, e1));
+                ms *= 3.f / (float)reps;
+            }
             if (ms < best) { best = ms; cfg = c; }
+            const char* v2 = std::getenv("CLG_TUNE_VERBOSE");
+            if (v2 && v2[0] == '2')  // every candidate
+                std::fprintf(stderr, "[clg tune]   candidate pin=%d block=%d xcd=%d: %.1f us\n", c.pm, c.block, c.xcd, ms * 1e3 / 3);
         }
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         const char* verbose = std::getenv("CLG_TUNE_VERBOSE");
-        if (verbose && verbose[0] == '1')
+        if (verbose && (verbose[0] == '1' || verbose[0] == '2'))
             std::fprintf(stderr, "[clg tune] staggered D prec=%d gprec=%d recon=%d mode=%d L=%dx%dx%dx%d -> block=%d xcd=%d pin=%d (%.1f us)\n",
                          prec, gprec, r12 ? 12 : 18, a.mode, a.g.L[0], a.g.L[1], a.g.L[2], a.g.L[3], cfg.block, cfg.xcd,
                          cfg.pm, best * 1e3 / 3);

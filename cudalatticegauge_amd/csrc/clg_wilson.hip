@@ -97,10 +97,12 @@ __global__ __launch_bounds__(256) void k_wilson_hop(HopArgs a) {
     typedef LinkIO<GP, RECON> LIO;
     constexpr bool STAGED = PM >= 5;
     constexpr int PMH = STAGED ? PM - 4 : PM;
-    const unsigned lw = a.tile_y > 0 ? tile_block(a.g, a.nblk, a.tile_y, a.tile_ymaj) : logical_wg(a.xcd);
+    const unsigned lw = STAGED && a.tile_y > 0 ? tile_block(a.g, a.nblk, a.tile_y, a.tile_ymaj) : logical_wg(a.xcd);
     for (int vs = 0; vs < a.spt; ++vs) {
     int p, h;
-    const bool valid = block_site(lw * (unsigned)a.spt + (unsigned)vs, a.g.Vh, a.nblk, a.pbase, a.pinter, p, h);
+    const bool valid = !STAGED && a.tile_y > 0
+                           ? tile64_site(a.g, a.nblk, a.pbase, a.tile_y, a.tile_ymaj, (int)threadIdx.x, p, h)
+                           : block_site(lw * (unsigned)a.spt + (unsigned)vs, a.g.Vh, a.nblk, a.pbase, a.pinter, p, h);
     const char* st = nullptr;
     const float* stn = nullptr;
     int hbase = 0;
@@ -157,19 +159,157 @@ __global__ __launch_bounds__(256) void k_wilson_hop(HopArgs a) {
     }
 }
 
+// ---- direction-split form
+// One site per thread walks a serial chain of eight dependent load-multiply groups, and a small lattice has
+// less than a wave per SIMD to hide it.  Here a workgroup of 8 waves takes 64 sites, one direction (mu,
+// forward or backward) per wave: the eight groups of a site run side by side, each wave leaves its
+// link-multiplied half-spinor (6 complex numbers a site) in LDS, and after one barrier waves 0..2 sum 4
+// spinor components each, rebuild the spin rows, add the x term and store.  All neighbours of a 64-site
+// block are then requested within one workgroup at one time, so what they share is still in the CU's L1 and
+// the XCD's L2: with the tiled order (tile64_site) it also leads on lattices that fill the chip.  Measured
+// (us, one site per thread -> split): FP64 D 8^4 7.6 -> 5.0, 24^3x24 101 -> 66, 32^4 311 -> 256; FP32 D
+// 24^3x48 95 -> 67; half hops FP64 16^4 11.7 -> 9.7, 32^4 154 -> 143 (non-temporal links), FP32 16^4 7.9 ->
+// 5.9, 24^3x48 49 -> 38.  It loses where one thread per site is already bound by memory with little state:
+// FP16 storage from 16^4 on (32^4 half hop 34 against 41), and FP64 D at 32^3x16 (122 against 125, staged).
+// The tuner times both.
+constexpr int kSplitSites = 64;
+
+// U h (forward) or U^dagger h (backward) of the neighbour in direction MU
+template <int MU, bool FWD, bool DAG, bool NTL, typename R, class SIO, class LIO>
+__device__ __forceinline__ void split_dir(const HopArgs& a, const Site& s, int p, int h, C2<R>* uh) {
+    C2<R> psi[12], hh[6], u[9];
+    const int Vh = a.g.Vh;
+    const Nbr n = FWD ? fwd_nbr<MU>(a.g, s, p) : bwd_nbr<MU>(a.g, s, p);
+    const unsigned pe = a.in_full ? (unsigned)n.p : 0u;
+    load_projected<SIO, MU, FWD != DAG ? 2 : 0>(a.in, a.inn, Vh, pe * SIO::NPL * Vh + n.h, pe * Vh + n.h, n.sign, psi, hh);
+    if constexpr (FWD) {
+        LIO::template load<NTL>(a.gauge, Vh, (unsigned)(p * 4 + MU) * LIO::NPL * Vh + h, u);
+        su3_mv(u, hh, uh);
+        su3_mv(u, hh + 3, uh + 3);
+    } else {
+        LIO::template load<NTL>(a.gauge, Vh, (unsigned)(n.p * 4 + MU) * LIO::NPL * Vh + n.h, u);
+        su3_mdv(u, hh, uh);
+        su3_mdv(u, hh + 3, uh + 3);
+    }
+}
+// spinor component K (spin K / 3, colour K % 3) of the hop in one direction, from its half-spinor in LDS
+template <int MU, int SG, int K, typename R>
+__device__ __forceinline__ C2<R> split_term(const C2<R>* half, int lane) {
+    constexpr int S = K / 3, C = K % 3;
+    constexpr int row = S == 2 ? G<MU, 2>::idx : S == 3 ? G<MU, 3>::idx : S;
+    constexpr int z = S == 2 ? G<MU, 2>::z + SG : S == 3 ? G<MU, 3>::z + SG : 0;
+    return mulz4<z>(half[(row * 3 + C) * kSplitSites + lane]);
+}
+template <int K, bool DAG, typename R>
+__device__ __forceinline__ C2<R> split_sum(const C2<R>* sm, int lane) {
+    constexpr int F = DAG ? 0 : 2, B = DAG ? 2 : 0, D = 6 * kSplitSites;
+    C2<R> v = split_term<0, F, K>(sm, lane);
+    v = cadd(v, split_term<0, B, K>(sm + D, lane));
+    v = cadd(v, split_term<1, F, K>(sm + 2 * D, lane));
+    v = cadd(v, split_term<1, B, K>(sm + 3 * D, lane));
+    v = cadd(v, split_term<2, F, K>(sm + 4 * D, lane));
+    v = cadd(v, split_term<2, B, K>(sm + 5 * D, lane));
+    v = cadd(v, split_term<3, F, K>(sm + 6 * D, lane));
+    return cadd(v, split_term<3, B, K>(sm + 7 * D, lane));
+}
+template <int W, bool DAG, typename R>
+__device__ __forceinline__ void split_sum4(const C2<R>* sm, int lane, C2<R>* v) {
+    v[0] = split_sum<4 * W, DAG>(sm, lane);
+    v[1] = split_sum<4 * W + 1, DAG>(sm, lane);
+    v[2] = split_sum<4 * W + 2, DAG>(sm, lane);
+    v[3] = split_sum<4 * W + 3, DAG>(sm, lane);
+}
+
+template <typename R, int SP, int GP, int RECON, bool DAG, bool HASX, bool NTL>
+__global__ __launch_bounds__(8 * kSplitSites) void k_wilson_hop_split(HopArgs a) {
+    typedef WilsonIO<SP> SIO;
+    typedef LinkIO<GP, RECON> LIO;
+    __shared__ C2<R> sm[8 * 6 * kSplitSites];
+    __shared__ float smax[SIO::SCALED ? 3 * kSplitSites : 1];
+    const int lane = (int)threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    int p, h;
+    const bool valid = a.tile_y > 0 ? tile64_site(a.g, a.nblk, a.pbase, a.tile_y, a.tile_ymaj, lane, p, h)
+                                    : block_site(logical_wg(a.xcd), kSplitSites, (unsigned)lane, a.g.Vh, a.nblk, a.pbase,
+                                                 a.pinter, p, h);
+    const unsigned po = a.out_full ? (unsigned)p : 0u;
+    const unsigned eo = po * SIO::NPL * a.g.Vh + h, no = po * a.g.Vh + h;
+    C2<R> xv[4];
+    if (valid) {
+        if constexpr (HASX)
+            if (w < 3) SIO::load4(a.x, a.xn, a.g.Vh, eo, no, w, xv);  // in flight beside the neighbour loads
+        const Site s = site_of(a.g, p, h);
+        C2<R> uh[6];
+        switch (w) {
+            case 0: split_dir<0, true, DAG, NTL, R, SIO, LIO>(a, s, p, h, uh); break;
+            case 1: split_dir<0, false, DAG, NTL, R, SIO, LIO>(a, s, p, h, uh); break;
+            case 2: split_dir<1, true, DAG, NTL, R, SIO, LIO>(a, s, p, h, uh); break;
+            case 3: split_dir<1, false, DAG, NTL, R, SIO, LIO>(a, s, p, h, uh); break;
+            case 4: split_dir<2, true, DAG, NTL, R, SIO, LIO>(a, s, p, h, uh); break;
+            case 5: split_dir<2, false, DAG, NTL, R, SIO, LIO>(a, s, p, h, uh); break;
+            case 6: split_dir<3, true, DAG, NTL, R, SIO, LIO>(a, s, p, h, uh); break;
+            default: split_dir<3, false, DAG, NTL, R, SIO, LIO>(a, s, p, h, uh); break;
+        }
+#pragma unroll
+        for (int k = 0; k < 6; ++k) sm[(w * 6 + k) * kSplitSites + lane] = uh[k];
+    }
+    __syncthreads();
+    C2<R> o[4];
+    if (w < 3 && valid) {
+        C2<R> acc[4];
+        if (w == 0) split_sum4<0, DAG>(sm, lane, acc);
+        else if (w == 1) split_sum4<1, DAG>(sm, lane, acc);
+        else split_sum4<2, DAG>(sm, lane, acc);
+        const C2<R> ca = cmk<R>((R)a.ar, (R)a.ai);
+        const C2<R> cb = cmk<R>((R)a.br, (R)a.bi);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if constexpr (HASX) {
+                o[k] = cmul(cb, xv[k]);
+                cfma(o[k], ca, acc[k]);
+            } else {
+                o[k] = cmul(ca, acc[k]);
+            }
+        }
+    }
+    if constexpr (SIO::SCALED) {  // the site scale is the largest of the three waves' components
+        if (w < 3 && valid) {
+            float m = 0.f;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) m = fmaxf(m, fmaxf(fabsf((float)o[k].x), fabsf((float)o[k].y)));
+            smax[w * kSplitSites + lane] = m;
+        }
+        __syncthreads();
+        if (w < 3 && valid) {
+            const float m = fmaxf(smax[lane], fmaxf(smax[kSplitSites + lane], smax[2 * kSplitSites + lane]));
+            const float inv = m > 0.f ? 1.0f / m : 0.f;
+            if (w == 0) a.outn[no] = m;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) o[k] = cscale(o[k], (R)inv);
+        }
+    }
+    if (w < 3 && valid) {
+        if (a.nt_out) SIO::template store4<R, true>(a.out, a.g.Vh, eo, w, o);
+        else SIO::store4(a.out, a.g.Vh, eo, w, o);
+    }
+}
+
 struct HopCfg {
     int pm;     // pin mode: 1 after each half of a direction, 2 after each direction; 3 / 4 the same
                 // with non-temporal link loads (links read once per launch stream past the caches);
-                // 5..8 as 1..4 with the z and t neighbours staged in LDS (block = L2*L3/2)
+                // 5..8 as 1..4 with the z and t neighbours staged in LDS (block = L2*L3/2);
+                // kSplitPm the direction-split kernel (block = kSplitSites sites, xcd 0 or 8)
     int block;  // threads per workgroup
     int xcd;    // 0: hardware order; 8: XCD-contiguous slabs, for full D with the two parities
                 // interleaved block by block; 1: XCD-contiguous slabs, parities one after the other;
                 // 10*TY + m (TY in 2, 4, 8; m = 0 x-major, 1 y-major): tiled plane schedule, staged
-                // launches only (clgd::tile_block), parities interleaved
+                // launches only (clgd::tile_block), parities interleaved; kSplitPm and kSplitNtPm take the same
+                // codes for the schedule in 64-site blocks (clgd::tile64_site), pm 1..4 take them + 100
     int spt = 1;  // sites per thread: consecutive logical blocks per workgroup (1, 2 or 4)
     int nt = 0;   // 1: the output spinor is stored with the non-temporal policy (it is not read again by
                   // the launch, so it need not take L2 space from the neighbour spinors and links)
 };
+constexpr int kTile64 = 100;  // tile64_site for one site per thread (pm 1..4, block 64)
 inline bool tiled_xcd(int xcd) { return xcd >= 20 && xcd <= 81 && (xcd / 10 == 2 || xcd / 10 == 4 || xcd / 10 == 8) && xcd % 10 <= 1; }
 
 template <typename R, int SP, int GP, int RECON, int PM>
@@ -184,6 +324,12 @@ void launch_pm(const HopArgs& a0, bool dag, bool hasx, hipStream_t st, int block
         a.tile_y = xcd / 10;
         a.tile_ymaj = xcd % 10;
         grid = (unsigned)(a.nblk * a.g.L[0] * a.g.L[1]);
+    } else if (tiled_xcd(xcd - kTile64)) {
+        a.xcd = 0;
+        a.spt = 1;
+        a.tile_y = (xcd - kTile64) / 10;
+        a.tile_ymaj = (xcd - kTile64) % 10;
+        grid = tile64_grid(a.g, a.nblk, a.tile_y);
     } else {
         a.xcd = xcd ? 8 : 0;
         a.pinter = xcd == 8 ? 1 : 0;
@@ -203,9 +349,37 @@ void launch_pm(const HopArgs& a0, bool dag, bool hasx, hipStream_t st, int block
     }
 }
 
+constexpr int kSplitPm = 9;    // the direction-split kernel
+constexpr int kSplitNtPm = 10;  // the same with non-temporal link loads
+inline bool split_pm(int pm) { return pm == kSplitPm || pm == kSplitNtPm; }
+template <typename R, int SP, int GP, int RECON, bool NTL>
+void launch_split(const HopArgs& a0, bool dag, bool hasx, hipStream_t st, int xcd, int nt) {
+    HopArgs a = a0;
+    a.nt_out = nt;
+    unsigned grid;
+    if (tiled_xcd(xcd)) {
+        a.tile_y = xcd / 10;
+        a.tile_ymaj = xcd % 10;
+        grid = tile64_grid(a.g, a.nblk, a.tile_y);
+    } else {
+        a.xcd = xcd ? 8 : 0;
+        a.pinter = xcd ? 1 : 0;
+        grid = sched_grid(a.g.Vh, a.nblk, kSplitSites, a.xcd, a.pinter);
+    }
+    if (dag) {
+        if (hasx) k_wilson_hop_split<R, SP, GP, RECON, true, true, NTL><<<grid, 8 * kSplitSites, 0, st>>>(a);
+        else k_wilson_hop_split<R, SP, GP, RECON, true, false, NTL><<<grid, 8 * kSplitSites, 0, st>>>(a);
+    } else {
+        if (hasx) k_wilson_hop_split<R, SP, GP, RECON, false, true, NTL><<<grid, 8 * kSplitSites, 0, st>>>(a);
+        else k_wilson_hop_split<R, SP, GP, RECON, false, false, NTL><<<grid, 8 * kSplitSites, 0, st>>>(a);
+    }
+}
+
 template <typename R, int SP, int GP, int RECON>
 int launch_t(const HopArgs& a, bool dag, bool hasx, hipStream_t st, HopCfg c) {
-    if (c.pm == 8) launch_pm<R, SP, GP, RECON, 8>(a, dag, hasx, st, c.block, c.xcd, c.spt, c.nt);
+    if (c.pm == kSplitPm) launch_split<R, SP, GP, RECON, false>(a, dag, hasx, st, c.xcd, c.nt);
+    else if (c.pm == kSplitNtPm) launch_split<R, SP, GP, RECON, true>(a, dag, hasx, st, c.xcd, c.nt);
+    else if (c.pm == 8) launch_pm<R, SP, GP, RECON, 8>(a, dag, hasx, st, c.block, c.xcd, c.spt, c.nt);
     else if (c.pm == 7) launch_pm<R, SP, GP, RECON, 7>(a, dag, hasx, st, c.block, c.xcd, c.spt, c.nt);
     else if (c.pm == 6) launch_pm<R, SP, GP, RECON, 6>(a, dag, hasx, st, c.block, c.xcd, c.spt, c.nt);
     else if (c.pm == 5) launch_pm<R, SP, GP, RECON, 5>(a, dag, hasx, st, c.block, c.xcd, c.spt, c.nt);
@@ -226,14 +400,14 @@ int staged_block(const Geo& g) {
 int launch_cfg(const HopArgs& a, int prec, int gprec, int recon, bool dag, bool hasx, hipStream_t st, HopCfg c) {
     // a staged launch needs one workgroup per (x,y) plane of one parity; the tuner only proposes
     // fitting ones, so a misfit comes from a forced configuration and is refused, not replaced
-    if (c.pm >= 5) {
+    if (c.pm >= 5 && c.pm <= 8) {
         const int sb = staged_block(a.g);
         CLG_CHECK_ARG(sb != 0 && c.block == sb,
                       "LDS-staged pin mode %d needs block = L2*L3/2 in {64,128,256} (lattice %dx%dx%dx%d gives %d), "
                       "asked for block %d",
                       c.pm, a.g.L[0], a.g.L[1], a.g.L[2], a.g.L[3], a.g.L[2] * a.g.L[3] / 2, c.block);
     }
-    if (tiled_xcd(c.xcd)) {
+    if (tiled_xcd(c.xcd) && !split_pm(c.pm)) {
         const int TY = c.xcd / 10, TX = 8 / TY;
         CLG_CHECK_ARG(c.pm >= 5 && c.spt == 1 && a.g.L[0] % TX == 0 && a.g.L[1] % TY == 0,
                       "tiled schedule %d needs an LDS-staged pin mode, one site per thread, L0 %% %d == 0 and "
@@ -284,6 +458,13 @@ bool valid_cfg(int pm, int blk, int xcd, int spt) {
     return pm >= 1 && pm <= 8 && (blk == 64 || blk == 128 || blk == 256) &&
            (xcd == 0 || xcd == 1 || xcd == 8 || tiled_xcd(xcd)) && (spt == 1 || spt == 2 || spt == 4);
 }
+// the configurations in 64-site blocks (the tuner's, its cache file's and CLG_TUNE_FORCE's): the
+// direction-split kernel, and one site per thread in the tiled order
+bool valid_split(int pm, int blk, int xcd, int spt) {
+    if (blk != kSplitSites || spt != 1) return false;
+    if (pm >= 1 && pm <= 4) return tiled_xcd(xcd - kTile64);
+    return split_pm(pm) && (xcd == 0 || xcd == 8 || tiled_xcd(xcd));
+}
 // process-wide overrides set through clg_autotune_enable / clg_autotune_force
 std::atomic<int> g_tune_mode{-1};  // -1: CLG_TUNE environment (default on), 0 off, 1 on
 std::atomic<int> g_forced{0};      // packed pin | block << 4 | xcd << 16 | spt << 24 | nt << 28, 0 = none
@@ -300,13 +481,20 @@ bool forced_cfg(HopCfg& c) {
     if (!e) return false;
     int pm = 0, blk = 0, xcd = 0, spt = 1, nt = 0;
     const int got = std::sscanf(e, "%d,%d,%d,%d,%d", &pm, &blk, &xcd, &spt, &nt);
-    if (got < 3 || !valid_cfg(pm, blk, xcd, spt) || (nt != 0 && nt != 1)) return false;
+    if (got < 3 || !(valid_cfg(pm, blk, xcd, spt) || valid_split(pm, blk, xcd, spt)) || (nt != 0 && nt != 1)) return false;
     c = HopCfg{pm, blk, xcd, spt, nt};
     return true;
 }
 
+// Untuned launches (tuning off, small lattices, graph capture) take the direction split up to this many
+// sites: measured, it is ahead of one site per thread for FP64 and FP32 spinors in the XCD-slab order up to
+// here (FP64 D at 24^3x16 48.6 against 61.2 us, FP32 26.7 against 27.7) and behind in FP16 from 16^4 on
+// (8.4 against 8.1 us).
+inline long split_default_max(int prec) { return prec == CLG_F16 ? 32768 : 262144; }
+
 int launch_hop(const HopArgs& a, int prec, int gprec, int recon, bool dag, bool hasx, hipStream_t st) {
-    const HopCfg dflt{1, 256, 8};
+    const long nsite = (long)a.nblk * a.g.Vh;
+    const HopCfg dflt = nsite <= split_default_max(prec) ? HopCfg{kSplitPm, kSplitSites, 8} : HopCfg{1, 256, 8};
     TuneKey k;
     std::memset(&k, 0, sizeof(k));
     k.prec = prec; k.gprec = gprec; k.recon = recon; k.dag = dag; k.hasx = hasx; k.nblk = a.nblk;
@@ -325,7 +513,8 @@ int launch_hop(const HopArgs& a, int prec, int gprec, int recon, bool dag, bool 
                 const std::vector<long>& v = e.first;
                 const std::vector<long>& c = e.second;
                 if (v.size() != 10 || (c.size() != 4 && c.size() != 5) ||
-                    !valid_cfg((int)c[0], (int)c[1], (int)c[2], (int)c[3]))
+                    !(valid_cfg((int)c[0], (int)c[1], (int)c[2], (int)c[3]) ||
+                      valid_split((int)c[0], (int)c[1], (int)c[2], (int)c[3])))
                     continue;
                 TuneKey t;
                 std::memset(&t, 0, sizeof(t));
@@ -345,9 +534,7 @@ int launch_hop(const HopArgs& a, int prec, int gprec, int recon, bool dag, bool 
     if (need_tune && tuning_enabled() && !aliased && cs == hipStreamCaptureStatusNone && (long)a.nblk * a.g.Vh >= 4096) {
         const HopCfg cands[] = {{1, 64, 0}, {1, 128, 0}, {1, 256, 0}, {2, 64, 0}, {2, 128, 0}, {2, 256, 0},
                                 {1, 64, 8}, {1, 128, 8}, {1, 256, 8}, {2, 64, 8}, {2, 128, 8}, {2, 256, 8},
-                                {3, 64, 8}, {3, 128, 8}, {3, 256, 8}, {4, 64, 8}, {4, 128, 8}, {4, 256, 8},
-                                {1, 128, 1}, {1, 256, 1}, {2, 128, 1}, {2, 256, 1},
-                                {3, 64, 1}, {3, 128, 1}, {3, 256, 1}, {4, 64, 1}, {4, 128, 1}, {4, 256, 1}};
+                                {3, 64, 8}, {3, 128, 8}, {3, 256, 8}, {4, 64, 8}, {4, 128, 8}, {4, 256, 8}};
         hipEvent_t e0, e1;
         CLG_HIP(hipEventCreate(&e0));
         CLG_HIP(hipEventCreate(&e1));
@@ -357,6 +544,18 @@ int launch_hop(const HopArgs& a, int prec, int gprec, int recon, bool dag, bool 
         for (int spt : {2, 4})
             for (int pm : {2, 4})
                 for (int blk : {128, 256}) all.push_back(HopCfg{pm, blk, 8, spt});
+        for (int pm : {kSplitPm, kSplitNtPm}) {
+            all.push_back(HopCfg{pm, kSplitSites, 8});
+            if (pm == kSplitPm) all.push_back(HopCfg{pm, kSplitSites, 0});
+            for (int TY : {2, 4, 8})
+                if (tile64_fits(a.g, TY))
+                    for (int m : {0, 1})
+                        for (int nt : {0, 1}) all.push_back(HopCfg{pm, kSplitSites, 10 * TY + m, 1, nt});
+        }
+        for (int TY : {2, 4, 8})
+            if (tile64_fits(a.g, TY))
+                for (int pm = 1; pm <= 4; ++pm)
+                    for (int nt : {0, 1}) all.push_back(HopCfg{pm, kSplitSites, kTile64 + 10 * TY, 1, nt});
         if (const int sb = staged_block(a.g)) {
             for (int pm = 5; pm <= 8; ++pm) all.push_back(HopCfg{pm, sb, 8});
             for (int pm : {6, 8}) all.push_back(HopCfg{pm, sb, 8, 2});
@@ -370,14 +569,18 @@ int launch_hop(const HopArgs& a, int prec, int gprec, int recon, bool dag, bool 
                         }
         }
         for (const HopCfg& c : all) {
-            if (c.xcd == 1 && a.nblk != 2) continue;  // one parity: the same launch as xcd 8
             CLG_TRY(launch_cfg(a, prec, gprec, recon, dag, hasx, st, c));  // warm
-            CLG_HIP(hipEventRecord(e0, st));
-            for (int r = 0; r < 3; ++r) CLG_TRY(launch_cfg(a, prec, gprec, recon, dag, hasx, st, c));
-            CLG_HIP(hipEventRecord(e1, st));
-            CLG_HIP(hipEventSynchronize(e1));
-            float ms = 0.f;
-            CLG_HIP(hipEventElapsedTime(&ms, e0, e1));
+            float ms = 0.f;  // of three launches
+            // a launch of a few microseconds is timed again over more of them: three are within the clock's noise
+            for (int reps : {3, 15}) {
+                if (reps == 15 && (ms > 0.12f || ms > 1.3f * best)) break;
+                CLG_HIP(hipEventRecord(e0, st));
+                for (int r = 0; r < reps; ++r) CLG_TRY(launch_cfg(a, prec, gprec, recon, dag, hasx, st, c));
+                CLG_HIP(hipEventRecord(e1, st));
+                CLG_HIP(hipEventSynchronize(e1));
+                CLG_HIP(hipEventElapsedTime(&ms, e0, e1));
+                ms *= 3.f / (float)reps;
+            }
             if (ms < best) { best = ms; cfg = c; }
             const char* v2 = std::getenv("CLG_TUNE_VERBOSE");
             if (v2 && v2[0] == '2')  // every candidate
