@@ -802,6 +802,11 @@ static int red_finish(clg_context ctx, unsigned nblk, int nr, double* out, int n
     return red_finish_at(ctx, ctx->red_partial, nblk, nr, out, nout, out2, cond, ref, eta, flag);
 }
 
+// the total of nblk one-value partials in ctx->red_partial, for other files' kernels
+int red_finish1(clg_context ctx, unsigned nblk, double* out) {
+    return red_finish(ctx, nblk, 1, out, 1, nullptr, nullptr, nullptr, 0.0, nullptr);
+}
+
 int blas_dot_dev(clg_context ctx, const clg_field_s* a, const clg_field_s* b, double* out) {
     CLG_TRY(check_pair(a, b));
     CLG_TRY(ensure_reduction_scratch(ctx, (size_t)kMaxRedGrid * (2 * kMaxK + 1)));

@@ -21,47 +21,80 @@ using namespace clgd;
 namespace clg {
 int blas_norm2_dev(clg_context, const clg_field_s*, double*);
 int fetch_doubles(clg_context, const double*, int, double*);
-int ensure_reduction_scratch(clg_context, size_t);
+int red_finish1(clg_context, unsigned, double*);
 int wilson_full(clg_context, clg_field_s*, const clg_field_s*, const clg_field_s*, double, bool, double, double);
 }  // namespace clg
 
 namespace {
 
 const int kBlk = 256;
-const int kMaxRedGrid = 2048;
 
-// r = a b^dagger, r = a^dagger b
+// r = a b^dagger
 __device__ __forceinline__ void su3_mmd(const cd* a, const cd* b, cd* r) {
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-            cd acc{0.0, 0.0};
-            acc = cadd(acc, cmul(a[3 * i], cconj(b[3 * j])));
-            acc = cadd(acc, cmul(a[3 * i + 1], cconj(b[3 * j + 1])));
-            acc = cadd(acc, cmul(a[3 * i + 2], cconj(b[3 * j + 2])));
+            cd acc = cmulc(b[3 * j], a[3 * i]);
+            cfmac(acc, b[3 * j + 1], a[3 * i + 1]);
+            cfmac(acc, b[3 * j + 2], a[3 * i + 2]);
             r[3 * i + j] = acc;
         }
 }
-__device__ __forceinline__ void su3_mdm(const cd* a, const cd* b, cd* r) {
+// r += a b^dagger, r += a^dagger b
+__device__ __forceinline__ void su3_mmd_add(const cd* a, const cd* b, cd* r) {
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            cd acc = cmulc(a[i], b[j]);
-            cfmac(acc, a[3 + i], b[3 + j]);
-            cfmac(acc, a[6 + i], b[6 + j]);
-            r[3 * i + j] = acc;
-        }
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) cfmac(r[3 * i + j], b[3 * j + k], a[3 * i + k]);
+}
+__device__ __forceinline__ void su3_mdm_add(const cd* a, const cd* b, cd* r) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) cfmac(r[3 * i + j], a[3 * k + i], b[3 * k + j]);
 }
 
-// (parity, half index) of the site with coordinates c (Lt even: h = lex / 2)
+// (parity, half index) of a site (Lt even: h = lex / 2), and one step along MU from site s as a change of
+// lexicographic index and of parity: steps along different directions add up
 struct PH {
     int p, h;
 };
-__device__ __forceinline__ PH ph_of(const Geo& g, const int* c) {
-    const int lex = ((c[0] * g.L[1] + c[1]) * g.L[2] + c[2]) * g.L[3] + c[3];
-    return PH{(c[0] + c[1] + c[2] + c[3]) & 1, lex >> 1};
+struct Step {
+    int dlex, flip;
+};
+template <int MU>
+__device__ __forceinline__ Step step_fwd(const Geo& g, const Site& s) {
+    const bool wrap = s.c[MU] == g.L[MU] - 1;
+    return Step{wrap ? -(g.L[MU] - 1) * g.stride[MU] : g.stride[MU], wrap ? 1 ^ (g.L[MU] & 1) : 1};
+}
+template <int MU>
+__device__ __forceinline__ Step step_bwd(const Geo& g, const Site& s) {
+    const bool wrap = s.c[MU] == 0;
+    return Step{wrap ? (g.L[MU] - 1) * g.stride[MU] : -g.stride[MU], wrap ? 1 ^ (g.L[MU] & 1) : 1};
+}
+__device__ __forceinline__ PH at_step(const Site& s, int p, Step a) { return PH{p ^ a.flip, (s.lex + a.dlex) >> 1}; }
+__device__ __forceinline__ PH at_steps(const Site& s, int p, Step a, Step b) {
+    return PH{p ^ a.flip ^ b.flip, (s.lex + a.dlex + b.dlex) >> 1};
+}
+// work order of the site kernels in 64-site blocks: the tiled plane order where it keeps the lanes busy
+// (neighbour planes then meet in one XCD's L2), else XCD slabs.  Gauge force at 32^3x16: eight tiles along y
+// 322 us, 2 x 4 tiles 341, 4 x 2 tiles 346, slabs 344; at 21x19x25x18, where a plane fills 4 of 3.5 blocks,
+// all within 1 %.
+struct SiteOrder {
+    int tile_y;  // 0: slabs
+    unsigned grid;
+};
+SiteOrder site_order(const Geo& g) {
+    if (tile64_fits(g, 8)) return SiteOrder{8, tile64_grid(g, 2, 8)};
+    return SiteOrder{0, sched_grid(g.Vh, 2, 64, 8, 1)};
+}
+__device__ __forceinline__ bool order_site(const Geo& g, int tile_y, int lane, int& p, int& h) {
+    return tile_y ? tile64_site(g, 2, 0, tile_y, 0, lane, p, h) : block_site(logical_wg(8), 64, (unsigned)lane, g.Vh, 2, 0, 1, p, h);
 }
 __device__ __forceinline__ void load_link(const char* U, const Geo& g, PH s, int mu, cd* m) {
     LinkIO<CLG_F64, 18>::load(U, g.Vh, (unsigned)((s.p * 4 + mu) * 9 * g.Vh + s.h), m);
@@ -153,16 +186,6 @@ __global__ void k_link_fill0(long n, double2* __restrict__ y) {
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
         y[i] = make_double2(0.0, 0.0);
 }
-__global__ __launch_bounds__(kRedBlock) void k_link_norm2(long n, const double2* __restrict__ x, double* partial,
-                                                          unsigned* counter, double* out) {
-    double v[1] = {0.0};
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        const double2 a = x[i];
-        v[0] += a.x * a.x + a.y * a.y;
-    }
-    reduce_finish<1>(v, partial, counter, out);
-}
-
 // U <- exp(a M) U per link (CFieldGaugeSU3::ExpMult, CFieldGaugeSU3.cu:452-490)
 __global__ __launch_bounds__(kBlk) void k_exp_mult(long nlink, int Vh, const char* M, char* U, double a, int prec) {
     const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -191,89 +214,145 @@ __global__ __launch_bounds__(kBlk) void k_normalize(long nlink, int Vh, char* U)
 }
 
 // sum over sites and mu < nu of (3 - ReTr U_mu(x) U_nu(x+mu) U_mu(x+nu)^dag U_nu(x)^dag)
-// (CFieldGaugeSU3.cu:308-371)
-__global__ __launch_bounds__(kRedBlock) void k_plaquette(Geo g, const char* U, double* partial, unsigned* counter,
-                                                         double* out) {
+// (CFieldGaugeSU3.cu:308-371).  A workgroup takes 64 sites, wave w two of the six planes (every direction
+// once: (0, w+1) and the other two), so a link a site needs for several planes comes from L1, and the partials
+// are summed by a second launch (a device-scope counter costs an L2 write-back per workgroup).  Measured at
+// 16^3x32: 37 us, against 67 with one thread per site, a counter and the planes in turn before.
+template <int MU, int NU>
+__device__ __forceinline__ double plaq_term(const Geo& g, const char* U, const Site& s, int p, int h) {
+    cd a[9], b[9], t[9], r[9];
+    load_link(U, g, PH{p, h}, MU, a);
+    load_link(U, g, at_step(s, p, step_fwd<MU>(g, s)), NU, b);
+    su3_mm(a, b, t);  // U_mu(x) U_nu(x+mu)
+    load_link(U, g, PH{p, h}, NU, a);
+    load_link(U, g, at_step(s, p, step_fwd<NU>(g, s)), MU, b);
+    su3_mm(a, b, r);  // U_nu(x) U_mu(x+nu)
+    double tr = 0.0;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) tr += t[k].x * r[k].x + t[k].y * r[k].y;  // ReTr t r^dag
+    return 3.0 - tr;
+}
+__global__ __launch_bounds__(192) void k_plaquette(Geo g, const char* U, double* partial, int tile_y) {
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    int p, h;
     double v[1] = {0.0};
-    for (long gid = (long)blockIdx.x * blockDim.x + threadIdx.x; gid < 2L * g.Vh;
-         gid += (long)gridDim.x * blockDim.x) {
-        const int p = (int)(gid / g.Vh), h = (int)(gid - (long)p * g.Vh);
+    if (order_site(g, tile_y, (int)threadIdx.x & 63, p, h)) {
         const Site s = site_of(g, p, h);
-        const PH x{p, h};
-        for (int mu = 0; mu < 4; ++mu) {
-            int cm[4] = {s.c[0], s.c[1], s.c[2], s.c[3]};
-            cm[mu] = cm[mu] + 1 == g.L[mu] ? 0 : cm[mu] + 1;
-            const PH xm = ph_of(g, cm);
-            cd umu[9];
-            load_link(U, g, x, mu, umu);
-            for (int nu = mu + 1; nu < 4; ++nu) {
-                int cn[4] = {s.c[0], s.c[1], s.c[2], s.c[3]};
-                cn[nu] = cn[nu] + 1 == g.L[nu] ? 0 : cn[nu] + 1;
-                const PH xn = ph_of(g, cn);
-                cd a[9], b[9], t1[9], t2[9];
-                load_link(U, g, xm, nu, a);
-                su3_mm(umu, a, t1);  // U_mu(x) U_nu(x+mu)
-                load_link(U, g, x, nu, a);
-                load_link(U, g, xn, mu, b);
-                su3_mm(a, b, t2);  // U_nu(x) U_mu(x+nu)
-                double tr = 0.0;
-                for (int k = 0; k < 9; ++k) tr += t1[k].x * t2[k].x + t1[k].y * t2[k].y;  // ReTr t1 t2^dag
-                v[0] += 3.0 - tr;
-            }
-        }
+        if (w == 0) v[0] = plaq_term<0, 1>(g, U, s, p, h) + plaq_term<2, 3>(g, U, s, p, h);
+        else if (w == 1) v[0] = plaq_term<0, 2>(g, U, s, p, h) + plaq_term<1, 3>(g, U, s, p, h);
+        else v[0] = plaq_term<0, 3>(g, U, s, p, h) + plaq_term<1, 2>(g, U, s, p, h);
     }
-    reduce_finish<1>(v, partial, counter, out);
+    block_partial<1>(v, partial);
 }
 
-// F_mu(x) += coef Ta[U_mu(x) C_mu(x)], C = sum_{nu != mu} U_nu(x+mu) U_mu(x+nu)^dag U_nu(x)^dag
-//                                            + U_nu(x+mu-nu)^dag U_mu(x-nu)^dag U_nu(x-nu)
-// (_kernelStapleAtSiteSU3CacheIndex + CActionGaugePlaquette force, CFieldGaugeSU3.cu:194-257)
-__global__ __launch_bounds__(kBlk) void k_gauge_force(Geo g, const char* U, char* F, double coef) {
-    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= 8L * g.Vh) return;
-    const int blk = (int)(gid / g.Vh), h = (int)(gid - (long)blk * g.Vh);
-    const int p = blk >> 2, mu = blk & 3;
-    const Site s = site_of(g, p, h);
-    const PH x{p, h};
-    int cpm[4] = {s.c[0], s.c[1], s.c[2], s.c[3]};
-    cpm[mu] = cpm[mu] + 1 == g.L[mu] ? 0 : cpm[mu] + 1;
-    const PH xpm = ph_of(g, cpm);
-    cd C[9];
-    for (int k = 0; k < 9; ++k) C[k] = cd{0.0, 0.0};
-    for (int nu = 0; nu < 4; ++nu) {
-        if (nu == mu) continue;
-        int cpn[4] = {s.c[0], s.c[1], s.c[2], s.c[3]};
-        cpn[nu] = cpn[nu] + 1 == g.L[nu] ? 0 : cpn[nu] + 1;
-        int cmn[4] = {s.c[0], s.c[1], s.c[2], s.c[3]};
-        cmn[nu] = cmn[nu] == 0 ? g.L[nu] - 1 : cmn[nu] - 1;
-        int cpmmn[4] = {cpm[0], cpm[1], cpm[2], cpm[3]};
-        cpmmn[nu] = cpmmn[nu] == 0 ? g.L[nu] - 1 : cpmmn[nu] - 1;
-        const PH xpn = ph_of(g, cpn), xmn = ph_of(g, cmn), xpmmn = ph_of(g, cpmmn);
-        cd a[9], b[9], t[9], r[9];
-        // upper staple
-        load_link(U, g, xpm, nu, a);
-        load_link(U, g, xpn, mu, b);
-        su3_mmd(a, b, t);
-        load_link(U, g, x, nu, a);
-        su3_mmd(t, a, r);
-        for (int k = 0; k < 9; ++k) C[k] = cadd(C[k], r[k]);
-        // lower staple: (U_mu(x-nu) U_nu(x+mu-nu))^dag U_nu(x-nu)
-        load_link(U, g, xmn, mu, a);
-        load_link(U, g, xpmmn, nu, b);
-        su3_mm(a, b, t);
-        load_link(U, g, xmn, nu, a);
-        su3_mdm(t, a, r);
-        for (int k = 0; k < 9; ++k) C[k] = cadd(C[k], r[k]);
+// A_mu(x) += step (coef Ta[U_mu(x) C_mu(x)]), C = sum_{nu != mu} U_nu(x+mu) U_mu(x+nu)^dag U_nu(x)^dag
+//                                                   + U_nu(x+mu-nu)^dag U_mu(x-nu)^dag U_nu(x-nu)
+// (_kernelStapleAtSiteSU3CacheIndex + CActionGaugePlaquette force, CFieldGaugeSU3.cu:194-257): the force
+// (step 1, A the force field) or, with A the momenta, force and momentum update in one pass.
+// A link reads 18 others (2.7 KB) for 432 compulsory bytes, and what bounds it is how many of those come
+// from past the 4 MB L2 (counters at 16^3x32: 360 MB fetched for 151 compulsory before the order and the
+// non-temporal policy below).  A workgroup takes 64 sites with wave mu on direction mu: U_nu(x) and
+// U_nu(x-nu), which three of the four waves need, are loaded once into LDS, the rest mostly meet in L1; the
+// order keeps neighbour planes in one XCD's L2, and A, which no other workgroup reads, is read and written
+// past it.  Measured at 16^3x32, us: one thread per link in parity-direction blocks 181, this kernel 80 (2.8
+// TB/s of compulsory bytes); without LDS staging 92 and without the non-temporal policy 90 in its 2 x 4 tile
+// form, which itself takes 84.
+// orders the staples: without it the compiler hoists the links of all six (256 VGPRs and spills)
+__device__ __forceinline__ void pin9(cd* C) {
+    asm volatile("" : "+v"(C[0].x), "+v"(C[0].y), "+v"(C[1].x), "+v"(C[1].y), "+v"(C[2].x), "+v"(C[2].y), "+v"(C[3].x),
+                 "+v"(C[3].y), "+v"(C[4].x), "+v"(C[4].y)::"memory");
+    asm volatile("" : "+v"(C[5].x), "+v"(C[5].y), "+v"(C[6].x), "+v"(C[6].y), "+v"(C[7].x), "+v"(C[7].y), "+v"(C[8].x),
+                 "+v"(C[8].y)::"memory");
+}
+// links of the workgroup's 64 sites in LDS: U_nu(x) and U_nu(x-nu), each needed by three of the four waves
+constexpr int kStageLinks = 4 * 9 * 64;  // per kind: [nu][matrix element][site]
+constexpr size_t kStageBytes = 2 * kStageLinks * sizeof(double2);
+__device__ __forceinline__ void stage_put(double2* sm, int nu, int lane, const cd* m) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) sm[(nu * 9 + k) * 64 + lane] = make_double2(m[k].x, m[k].y);
+}
+__device__ __forceinline__ void stage_get(const double2* sm, int nu, int lane, cd* m) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+        const double2 v = sm[(nu * 9 + k) * 64 + lane];
+        m[k] = cd{v.x, v.y};
     }
-    cd u[9], f[9];
-    load_link(U, g, x, mu, u);
+}
+template <int MU, int NU>
+__device__ __forceinline__ void add_staples(const Geo& g, const char* U, const double2* sm, const Site& s, int p, int lane,
+                                            Step fm, cd* C) {
+    if constexpr (MU != NU) {
+        const Step fn = step_fwd<NU>(g, s), bn = step_bwd<NU>(g, s);
+        cd a[9], b[9], t[9];
+        load_link(U, g, at_step(s, p, fm), NU, a);
+        load_link(U, g, at_step(s, p, fn), MU, b);
+        su3_mmd(a, b, t);
+        stage_get(sm, NU, lane, a);
+        su3_mmd_add(t, a, C);
+        pin9(C);
+        // lower staple: (U_mu(x-nu) U_nu(x+mu-nu))^dag U_nu(x-nu)
+        load_link(U, g, at_step(s, p, bn), MU, a);
+        load_link(U, g, at_steps(s, p, fm, bn), NU, b);
+        su3_mm(a, b, t);
+        stage_get(sm + kStageLinks, NU, lane, a);
+        su3_mdm_add(t, a, C);
+        pin9(C);
+    }
+}
+// f = Ta[U_mu(x) C_mu(x)], u = U_mu(x)
+template <int MU>
+__device__ __forceinline__ void plaquette_force(const Geo& g, const char* U, const double2* sm, const Site& s, int p,
+                                                int lane, cd* u, cd* f) {
+    const Step fm = step_fwd<MU>(g, s);
+    cd C[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) C[k] = cd{0.0, 0.0};
+    add_staples<MU, 0>(g, U, sm, s, p, lane, fm, C);
+    add_staples<MU, 1>(g, U, sm, s, p, lane, fm, C);
+    add_staples<MU, 2>(g, U, sm, s, p, lane, fm, C);
+    add_staples<MU, 3>(g, U, sm, s, p, lane, fm, C);
+    stage_get(sm, MU, lane, u);
     su3_mm(u, C, f);
     su3_ta(f);
-    const unsigned e = (unsigned)(blk * 9 * g.Vh + h);
+}
+// U_mu(x) and U_mu(x-mu) of this wave's direction into LDS
+template <int MU>
+__device__ __forceinline__ void stage_links(const Geo& g, const char* U, double2* sm, const Site& s, int p, int h, int lane) {
+    cd a[9], b[9];
+    load_link(U, g, PH{p, h}, MU, a);
+    load_link(U, g, at_step(s, p, step_bwd<MU>(g, s)), MU, b);
+    stage_put(sm, MU, lane, a);
+    stage_put(sm + kStageLinks, MU, lane, b);
+}
+__global__ __launch_bounds__(kBlk) void k_gauge_force(Geo g, const char* U, char* A, double coef, double step, int tile_y) {
+    extern __shared__ double2 sm[];
+    const int mu = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+    int p, h;
+    const bool valid = order_site(g, tile_y, lane, p, h);
+    const Site s = site_of(g, p, valid ? h : 0);
+    if (valid) {
+        switch (mu) {
+            case 0: stage_links<0>(g, U, sm, s, p, h, lane); break;
+            case 1: stage_links<1>(g, U, sm, s, p, h, lane); break;
+            case 2: stage_links<2>(g, U, sm, s, p, h, lane); break;
+            default: stage_links<3>(g, U, sm, s, p, h, lane); break;
+        }
+    }
+    __syncthreads();
+    if (!valid) return;
+    cd u[9], f[9];
+    switch (mu) {
+        case 0: plaquette_force<0>(g, U, sm, s, p, lane, u, f); break;
+        case 1: plaquette_force<1>(g, U, sm, s, p, lane, u, f); break;
+        case 2: plaquette_force<2>(g, U, sm, s, p, lane, u, f); break;
+        default: plaquette_force<3>(g, U, sm, s, p, lane, u, f); break;
+    }
+    const unsigned e = (unsigned)((p * 4 + mu) * 9 * g.Vh + h);
     cd cur[9];
-    LinkIO<CLG_F64, 18>::load(F, g.Vh, e, cur);
-    for (int k = 0; k < 9; ++k) cur[k] = cd{cur[k].x + coef * f[k].x, cur[k].y + coef * f[k].y};
-    LinkIO<CLG_F64, 18>::store(F, g.Vh, e, cur);
+    LinkIO<CLG_F64, 18>::load<true>(A, g.Vh, e, cur);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) cur[k] = cd{cur[k].x + step * (coef * f[k].x), cur[k].y + step * (coef * f[k].y)};
+    LinkIO<CLG_F64, 18>::store<true>(A, g.Vh, e, cur);
 }
 
 int check_link_field(const clg_field_s* f, const char* what) {
@@ -286,12 +365,6 @@ unsigned ew_grid(clg_context ctx, long n) {
     const long g = (n + kBlk - 1) / kBlk, cap = (long)ctx->num_cu * 16;
     return (unsigned)std::max<long>(1, std::min(g, cap));
 }
-unsigned red_grid(clg_context ctx, long n) {
-    const long g = (n + kRedBlock * 4 - 1) / (kRedBlock * 4);
-    const long cap = std::min<long>(kMaxRedGrid, (long)ctx->num_cu * 4);
-    return (unsigned)std::max<long>(1, std::min(g, cap));
-}
-
 }  // namespace
 
 // ================================================================ host building blocks
@@ -309,15 +382,6 @@ int link_zero(clg_context ctx, clg_field_s* y) {
     CLG_HIP(hipGetLastError());
     return CLG_OK;
 }
-int link_norm2_dev(clg_context ctx, const clg_field_s* x, double* out) {
-    const long n = link_values(x);
-    const unsigned g = red_grid(ctx, n);
-    CLG_TRY(ensure_reduction_scratch(ctx, (size_t)g));
-    k_link_norm2<<<g, kRedBlock, 0, ctx->stream>>>(n, (const double2*)x->data, ctx->red_partial, ctx->red_counter,
-                                                    out);
-    CLG_HIP(hipGetLastError());
-    return CLG_OK;
-}
 int exp_mult(clg_context ctx, const clg_field_s* M, clg_field_s* U, double a, int prec) {
     const long n = 8L * U->Vh;
     k_exp_mult<<<grid_for(n, kBlk), kBlk, 0, ctx->stream>>>(n, (int)U->Vh, (const char*)M->data, (char*)U->data, a,
@@ -325,21 +389,22 @@ int exp_mult(clg_context ctx, const clg_field_s* M, clg_field_s* U, double a, in
     CLG_HIP(hipGetLastError());
     return CLG_OK;
 }
-int gauge_force(clg_context ctx, clg_field_s* F, const clg_field_s* U, double beta) {
+// A += step (force of the plaquette action)
+int gauge_force(clg_context ctx, clg_field_s* A, const clg_field_s* U, double beta, double step) {
     const Geo g = make_geo(U);
-    k_gauge_force<<<grid_for(8L * g.Vh, kBlk), kBlk, 0, ctx->stream>>>(g, (const char*)U->data, (char*)F->data,
-                                                                        -beta / 6.0);
+    const SiteOrder o = site_order(g);
+    CLG_HIP(hipFuncSetAttribute((const void*)k_gauge_force, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kStageBytes));
+    k_gauge_force<<<o.grid, kBlk, kStageBytes, ctx->stream>>>(g, (const char*)U->data, (char*)A->data, -beta / 6.0, step, o.tile_y);
     CLG_HIP(hipGetLastError());
     return CLG_OK;
 }
 int plaquette_dev(clg_context ctx, const clg_field_s* U, double* out) {
     const Geo g = make_geo(U);
-    const unsigned grid = red_grid(ctx, 2L * g.Vh * 6);
-    CLG_TRY(ensure_reduction_scratch(ctx, (size_t)grid));
-    k_plaquette<<<grid, kRedBlock, 0, ctx->stream>>>(g, (const char*)U->data, ctx->red_partial, ctx->red_counter,
-                                                     out);
+    const SiteOrder o = site_order(g);
+    CLG_TRY(ensure_reduction_scratch(ctx, (size_t)o.grid));
+    k_plaquette<<<o.grid, 192, 0, ctx->stream>>>(g, (const char*)U->data, ctx->red_partial, o.tile_y);
     CLG_HIP(hipGetLastError());
-    return CLG_OK;
+    return red_finish1(ctx, o.grid, out);
 }
 
 }  // namespace clg
@@ -388,10 +453,18 @@ struct Integrator {
     std::vector<clg_field_s*> xcache;  // Wilson: last (DD^dagger)^-1 phi, the next solve's start
     clg_hmc_report* rep;
 
+    // P += step F(gauge actions), without a force field
+    int gauge_update_p(double step) {
+        for (int i = 0; i < nact; ++i)
+            if (acts[i].kind == CLG_ACTION_GAUGE_PLAQUETTE) CLG_TRY(gauge_force(ctx, P, U, acts[i].beta, step));
+        if (rep) rep->force_evaluations++;
+        return CLG_OK;
+    }
+    // F += force of the gauge or the fermion actions
     int force_into(bool fermion) {
         for (int i = 0; i < nact; ++i) {
             const clg_action& a = acts[i];
-            if (!fermion && a.kind == CLG_ACTION_GAUGE_PLAQUETTE) CLG_TRY(gauge_force(ctx, F, U, a.beta));
+            if (!fermion && a.kind == CLG_ACTION_GAUGE_PLAQUETTE) CLG_TRY(gauge_force(ctx, F, U, a.beta, 1.0));
             if (!fermion) continue;
             clg_solve_report r{};
             int st = CLG_OK;
@@ -415,16 +488,19 @@ struct Integrator {
     }
     // UpdatePF / UpdatePG: P += step F(fermion or gauge actions)
     int update_p(double step, bool fermion) {
+        if (!fermion) return gauge_update_p(step);
         CLG_TRY(link_zero(ctx, F));
         CLG_TRY(force_into(fermion));
         return link_axpy(ctx, P, step, F);
     }
     // all actions in one force (CIntegrator::UpdateP, CIntegrator.cpp:219-242)
     int update_p_all(double step) {
-        CLG_TRY(link_zero(ctx, F));
-        CLG_TRY(force_into(false));
-        CLG_TRY(force_into(true));
-        return link_axpy(ctx, P, step, F);
+        CLG_TRY(gauge_update_p(step));
+        if (!has(true)) {
+            if (rep) rep->force_evaluations++;
+            return CLG_OK;
+        }
+        return update_p(step, true);
     }
     // ZeroForce, force, PreserveFields, AddForceToFieldDirectly(fg), Update(step), RecoverFields
     int fg_update(double fg, double step, bool fermion) {
@@ -485,7 +561,7 @@ struct Integrator {
     // CIntegrator::GetEnergy (CIntegrator.cpp:256-279): kinetic + every action, FP64
     int energy(double* total, double* kin, double* per_action) {
         double* dv = ctx->red_result + 40;
-        CLG_TRY(link_norm2_dev(ctx, P, dv));
+        CLG_TRY(blas_norm2_dev(ctx, P, dv));
         CLG_TRY(fetch_doubles(ctx, dv, 1, kin));
         double sum = *kin;
         for (int i = 0; i < nact; ++i) {
@@ -596,7 +672,7 @@ int clg_gauge_kinetic_energy(clg_context ctx, clg_field P, double* out) {
     CLG_CHECK_ARG(ctx && out, "null argument");
     CLG_TRY(check_link_field(P, "momentum"));
     (void)hipSetDevice(ctx->device);
-    CLG_TRY(link_norm2_dev(ctx, P, ctx->red_result + 40));
+    CLG_TRY(blas_norm2_dev(ctx, P, ctx->red_result + 40));
     return fetch_doubles(ctx, ctx->red_result + 40, 1, out);
 }
 
@@ -648,7 +724,7 @@ int clg_gauge_force(clg_context ctx, clg_field force, clg_field gauge, double be
     CLG_TRY(check_same_lattice(force, gauge));
     CLG_CHECK_ARG(force != gauge, "force and gauge must differ");
     (void)hipSetDevice(ctx->device);
-    return gauge_force(ctx, force, gauge, beta);
+    return gauge_force(ctx, force, gauge, beta, 1.0);
 }
 
 // CFieldFermionWilsonSquareSU3::PrepareForHMCS (CFieldFermionWilsonSquareSU3.cu:867-906): phi = D eta

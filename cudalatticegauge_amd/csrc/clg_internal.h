@@ -73,10 +73,9 @@ struct clg_context_s {
     hipStream_t stream = nullptr;
     int num_cu = 0;
     char arch[64] = {0};
-    // reduction scratch: per-block partials, a done-counter, device results
+    // reduction scratch: per-block partials, device results
     double* red_partial = nullptr;
     size_t red_partial_cap = 0;  // doubles
-    unsigned* red_counter = nullptr;
     double* red_result = nullptr;  // 4096 doubles of device-resident results
     double* host_result = nullptr;  // pinned
     // solver workspace (Hessenberg, Givens, scalars), grow-only
@@ -758,9 +757,10 @@ template <> struct LinkIO<CLG_F64, 18> {
 #pragma unroll
         for (int k = 0; k < 9; ++k) { const double2 a = ldq<double2, NT>(b, Vh, k, e); m[k] = C2<R>{(R)a.x, (R)a.y}; }
     }
+    template <bool NT = false>
     __device__ __forceinline__ static void store(char* b, int Vh, unsigned e, const cd* m) {
 #pragma unroll
-        for (int k = 0; k < 9; ++k) stp<double2>(b, Vh, k, e, make_double2(m[k].x, m[k].y));
+        for (int k = 0; k < 9; ++k) stq<double2, NT>(b, Vh, k, e, make_double2(m[k].x, m[k].y));
     }
 };
 template <> struct LinkIO<CLG_F64, 12> {
@@ -1019,64 +1019,6 @@ __device__ void block_partial(double (&v)[NR], double* partial) {
         for (int w = 0; w < nw; ++w) s += sm[w][r];
         partial[(size_t)blockIdx.x * NR + r] = s;
     }
-}
-
-// Reduce NR per-lane FP64 values over the grid (blockDim.x <= kRedBlock, a multiple of 64);
-// the last workgroup to finish writes out[0..NR), resets the counter and returns true on its
-// thread 0.  partial holds gridDim.x * NR doubles.
-template <int NR>
-__device__ bool reduce_finish(double (&v)[NR], double* partial, unsigned* counter, double* out) {
-    __shared__ double sm[kRedBlock / 64][NR];
-    __shared__ int is_last;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int nw = blockDim.x >> 6;
-#pragma unroll
-    for (int r = 0; r < NR; ++r) v[r] = wave_sum(v[r]);
-    if (lane == 0) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) sm[wv][r] = v[r];
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int r = 0; r < NR; ++r) {
-            double s = 0;
-            for (int w = 0; w < nw; ++w) s += sm[w][r];
-            partial[(size_t)blockIdx.x * NR + r] = s;
-        }
-        __threadfence();
-        const unsigned t = atomicAdd(counter, 1u);
-        is_last = (t == gridDim.x - 1);
-    }
-    __syncthreads();
-    if (!is_last) return false;
-    // acquire: the fence invalidates this CU's vector L1, so the plain loads below see every
-    // block's partials (each published by a release fence before its counter increment)
-    __threadfence();
-    double acc[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) acc[r] = 0;
-    for (int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) acc[r] += partial[(size_t)b * NR + r];
-    }
-#pragma unroll
-    for (int r = 0; r < NR; ++r) acc[r] = wave_sum(acc[r]);
-    __syncthreads();
-    if (lane == 0) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) sm[wv][r] = acc[r];
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int r = 0; r < NR; ++r) {
-            double s = 0;
-            for (int w = 0; w < nw; ++w) s += sm[w][r];
-            out[r] = s;
-        }
-        *counter = 0u;
-        return true;
-    }
-    return false;
 }
 
 }  // namespace clgd

@@ -476,8 +476,6 @@ int init_context(clg_context c) {
     c->num_cu = prop.multiProcessorCount;
     std::snprintf(c->arch, sizeof(c->arch), "%s", prop.gcnArchName);
     CLG_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-    CLG_HIP(hipMalloc((void**)&c->red_counter, 64 * sizeof(unsigned)));
-    CLG_HIP(hipMemsetAsync(c->red_counter, 0, 64 * sizeof(unsigned), c->stream));
     CLG_HIP(hipMalloc((void**)&c->red_result, 4096 * sizeof(double)));
     CLG_HIP(hipHostMalloc((void**)&c->host_result, 4096 * sizeof(double), hipHostMallocDefault));
     CLG_HIP(hipEventCreate(&c->ev0));
@@ -521,7 +519,6 @@ int clg_finalize(clg_context c) {
     for (clg_field_s* f : c->scratch) clg_field_destroy(f);
     c->scratch.clear();
     if (c->red_partial) (void)hipFree(c->red_partial);
-    if (c->red_counter) (void)hipFree(c->red_counter);
     if (c->red_result) (void)hipFree(c->red_result);
     if (c->host_result) (void)hipHostFree(c->host_result);
     if (c->ws) (void)hipFree(c->ws);
