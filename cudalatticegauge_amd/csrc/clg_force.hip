@@ -13,6 +13,7 @@
 //   phi_i = (D D^dagger + b_i)^-1 phi, d_i = D0 phi_i (massless),
 //   F_mu(x) -= Ta[ a_i eta_mu(x) s ( (U phi_i(x+mu)) d_i(x)^dagger + phi_i(x) (U d_i(x+mu))^dagger ) ]
 #include "clg_internal.h"
+#include "clg_wilson_common.h"
 
 #include <chrono>
 #include <cmath>
@@ -34,132 +35,161 @@ namespace {
 
 typedef C2<double> cx;
 
-// gamma_mu rows (chiral set, GammaMatrix.h:447-475): (g psi)[r] = i^z[r] psi[idx[r]]
-__constant__ int kGIdx[4][4] = {{3, 2, 1, 0}, {3, 2, 1, 0}, {2, 3, 0, 1}, {2, 3, 0, 1}};
-__constant__ int kGZ4[4][4] = {{3, 3, 1, 1}, {2, 0, 0, 2}, {3, 1, 1, 3}, {0, 0, 0, 0}};
-__device__ __forceinline__ cx mulz4r(cx a, int k) {
-    switch (k & 3) {
-        case 1: return cx{-a.y, a.x};
-        case 2: return cx{-a.x, -a.y};
-        case 3: return cx{a.y, -a.x};
-        default: return a;
-    }
-}
-// out = (1 + sg gamma_mu) psi   (sg = +1 or -1)
-__device__ __forceinline__ void proj_full(const cx* psi, int mu, int sg, cx* out) {
-    for (int r = 0; r < 4; ++r) {
-        const int src = kGIdx[mu][r];
-        const int z = kGZ4[mu][r] + (sg < 0 ? 2 : 0);
-        for (int c = 0; c < 3; ++c) out[3 * r + c] = cadd(psi[3 * r + c], mulz4r(psi[3 * src + c], z));
-    }
-}
-
+// F(e) += f m, F read and written past L2: no other workgroup reads it
 __device__ __forceinline__ void add_link(char* F, int Vh, unsigned e, const cx* m, double f) {
     cx cur[9];
-    LinkIO<CLG_F64, 18>::load(F, Vh, e, cur);
+    LinkIO<CLG_F64, 18>::load<true>(F, Vh, e, cur);
+#pragma unroll
     for (int k = 0; k < 9; ++k) cur[k] = cx{cur[k].x + f * m[k].x, cur[k].y + f * m[k].y};
-    LinkIO<CLG_F64, 18>::store(F, Vh, e, cur);
+    LinkIO<CLG_F64, 18>::store<true>(F, Vh, e, cur);
+}
+// m += a b^dagger on colour vectors
+__device__ __forceinline__ void outer_add(const cx* a, const cx* b, cx* m) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) cfmac(m[3 * i + j], b[j], a[i]);
 }
 
-// Launch shape of the force kernels: 128-thread workgroups (the register budget that fits their
-// per-site state without spilling), XCD-contiguous slabs with the parities interleaved block by
-// block, so the x+mu neighbour reads of one parity meet the site reads of the other in one L2.
-constexpr int kForceBlock = 128;
+// The force kernels run in 64-site blocks, wave mu of a workgroup on direction mu (clg::site_order): the
+// site's own vectors, which all four waves read, come from L1, and there are four times the waves of one
+// thread per site.
 
-// Wilson force kernel; X = (DD^dagger)^-1 phi ("left"), Y = D^dagger X ("right"), FULL FP64 fields
-__global__ __launch_bounds__(kForceBlock) void k_wilson_force(Geo g, const char* X, const char* Y, const char* U, char* F,
-                                                              double kappa) {
-    int p, h;
-    if (!map_site(g.Vh, 2, 0, 8, 1, p, h)) return;
-    const Site s = site_of(g, p, h);
+// half-spinor (1 + s g_mu) psi, rows 0 and 1
+template <int MU, int SG>
+__device__ __forceinline__ void load_half(const char* f, int Vh, int p, int h, cx* hh) {
+    cx psi[12];
+    WilsonIO<CLG_F64>::load(f, nullptr, Vh, (unsigned)(p * 12 * Vh + h), 0u, psi);
+    project<MU, SG>(psi, hh);
+}
+// Wilson force kernel; X = (DD^dagger)^-1 phi, Y = D^dagger X, FULL FP64 fields.  (1 -+ g_mu) has rank 2 and is
+// twice a projector, so the spin sum over four rows of ((1-g_mu) Y(x+mu)) X(x)^dagger is the sum over rows 0
+// and 1 of both vectors' half-spinors, and the same for the other term: half the products, and 24 complex
+// numbers a lane instead of 48.  Bound by HBM: measured at 32^3x16 215 us, 5.1 TB/s of the 1.1 GB compulsory
+// bytes (one thread per site, four rows, everything through L2: 304 us).
+template <int MU>
+__device__ __forceinline__ void wilson_force_mu(const Geo& g, const Site& s, int p, int h, const char* X, const char* Y,
+                                                const char* U, char* F, double kappa) {
     const int Vh = g.Vh;
-    cx xl[12], xr[12];
-    WilsonIO<CLG_F64>::load(X, nullptr, Vh, (unsigned)(p * 12 * Vh + h), 0u, xl);
-    WilsonIO<CLG_F64>::load(Y, nullptr, Vh, (unsigned)(p * 12 * Vh + h), 0u, xr);
-    for (int mu = 0; mu < 4; ++mu) {
-        Nbr n;
-        switch (mu) {
-            case 0: n = fwd_nbr<0>(g, s, p); break;
-            case 1: n = fwd_nbr<1>(g, s, p); break;
-            case 2: n = fwd_nbr<2>(g, s, p); break;
-            default: n = fwd_nbr<3>(g, s, p); break;
-        }
-        cx pr[12], pl[12], r1[12], r2[12];
-        WilsonIO<CLG_F64>::load(Y, nullptr, Vh, (unsigned)(n.p * 12 * Vh + n.h), 0u, pr);
-        WilsonIO<CLG_F64>::load(X, nullptr, Vh, (unsigned)(n.p * 12 * Vh + n.h), 0u, pl);
-        proj_full(pr, mu, -1, r1);  // (1 - g_mu) Y(x+mu)
-        proj_full(xr, mu, +1, r2);  // (1 + g_mu) Y(x)
-        // mid[3a+c] = sum_s r1_s[a] conj(xl_s[c]) + pl_s[a] conj(r2_s[c])   (makeSU3Contract, SU3.h:395-503)
-        cx mid[9];
-        for (int a = 0; a < 3; ++a)
-            for (int c = 0; c < 3; ++c) {
-                cx acc{0.0, 0.0};
-                for (int sp = 0; sp < 4; ++sp) {
-                    cfmac(acc, xl[3 * sp + c], r1[3 * sp + a]);
-                    cfmac(acc, r2[3 * sp + c], pl[3 * sp + a]);
-                }
-                mid[3 * a + c] = acc;
-            }
-        cx u[9], f[9];
-        const unsigned el = (unsigned)((p * 4 + mu) * 9 * Vh + h);
-        LinkIO<CLG_F64, 18>::load(U, Vh, el, u);
-        su3_mm(u, mid, f);
-        su3_ta(f);
-        add_link(F, Vh, el, f, n.sign < 0 ? -kappa : kappa);
+    const Nbr n = fwd_nbr<MU>(g, s, p);
+    const unsigned el = (unsigned)((p * 4 + MU) * 9 * Vh + h);
+    cx a[6], b[6], mid[9], u[9], f[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) mid[k] = cx{0.0, 0.0};
+    load_half<MU, 2>(Y, Vh, n.p, n.h, a);
+    load_half<MU, 2>(X, Vh, p, h, b);
+    outer_add(a, b, mid);
+    outer_add(a + 3, b + 3, mid);
+    load_half<MU, 0>(X, Vh, n.p, n.h, a);
+    load_half<MU, 0>(Y, Vh, p, h, b);
+    outer_add(a, b, mid);
+    outer_add(a + 3, b + 3, mid);
+    LinkIO<CLG_F64, 18>::load<true>(U, Vh, el, u);
+    su3_mm(u, mid, f);
+    su3_ta(f);
+    add_link(F, Vh, el, f, n.sign < 0 ? -kappa : kappa);
+}
+__global__ __launch_bounds__(256) void k_wilson_force(Geo g, const char* X, const char* Y, const char* U, char* F,
+                                                      double kappa, int tile_y) {
+    const int mu = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    int p, h;
+    if (!order_site(g, tile_y, (int)threadIdx.x & 63, p, h)) return;
+    const Site s = site_of(g, p, h);
+    switch (mu) {
+        case 0: wilson_force_mu<0>(g, s, p, h, X, Y, U, F, kappa); break;
+        case 1: wilson_force_mu<1>(g, s, p, h, X, Y, U, F, kappa); break;
+        case 2: wilson_force_mu<2>(g, s, p, h, X, Y, U, F, kappa); break;
+        default: wilson_force_mu<3>(g, s, p, h, X, Y, U, F, kappa); break;
     }
 }
 
-// staggered force kernel over npole (phi_i, d_i) pairs with numerators a_i
+// staggered force kernel over npole (phi_i, d_i) pairs with numerators a_i.  The link does not depend on the
+// pole, so the poles' outer products are summed first,
+//   sum_i a_i [ (U phi_i(x+mu)) d_i(x)^dagger + phi_i(x) (U d_i(x+mu))^dagger ] = U M1 + M2 U^dagger,
+// and U and Ta are applied once: 84 instead of 210 FP64 operations per pole and link.  Bound by the loads in
+// flight (172 VGPRs, two waves per SIMD; at most 168 spills and is no faster) and by L2: the site's own
+// vectors are read once per workgroup, two poles a round, through LDS (straight from L1/L2 by all four
+// waves: 113 us), the next round's in flight during this one.  Measured: 24^3x8, 12 poles 143 -> 83 us;
+// 12x10x14x16, 3 poles 31 -> 14; 19x21x15x18, 1 pole 54 -> 42 (one thread per site, the four directions and
+// the whole expression per pole in turn before).
 struct PolePtrs {
     const char* phi[32];
     const char* d[32];
     double a[32];
 };
-__global__ __launch_bounds__(kForceBlock) void k_ks_force(Geo g, PolePtrs pp, int npole, const char* U, char* F) {
-    int p, h;
-    if (!map_site(g.Vh, 2, 0, 8, 1, p, h)) return;
-    const Site s = site_of(g, p, h);
+__global__ __launch_bounds__(256) void k_ks_force(Geo g, PolePtrs pp, int npole, const char* U, char* F, int tile_y) {
+    // two poles a round: own vectors [buffer][pole, phi or d][colour][site], already times a_i
+    __shared__ double2 own[2][4][3][64];
+    const int mu = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
     const int Vh = g.Vh;
-    for (int mu = 0; mu < 4; ++mu) {
-        Nbr n;
-        switch (mu) {
-            case 0: n = fwd_nbr<0>(g, s, p); break;
-            case 1: n = fwd_nbr<1>(g, s, p); break;
-            case 2: n = fwd_nbr<2>(g, s, p); break;
-            default: n = fwd_nbr<3>(g, s, p); break;
-        }
-        int sum = 0;
-        for (int nu = 0; nu < mu; ++nu) sum += s.c[nu];
-        const double eta = (sum & 1) ? -1.0 : 1.0;
-        cx u[9];
-        const unsigned el = (unsigned)((p * 4 + mu) * 9 * Vh + h);
-        LinkIO<CLG_F64, 18>::load(U, Vh, el, u);
-        cx tot[9];
-        for (int k = 0; k < 9; ++k) tot[k] = cx{0.0, 0.0};
-        for (int r = 0; r < npole; ++r) {
-            cx phin[3], dn[3], phix[3], dx[3], t1[3], t2[3];
-            KSIO<CLG_F64>::load(pp.phi[r], nullptr, Vh, (unsigned)(n.p * 3 * Vh + n.h), 0u, phin);
-            KSIO<CLG_F64>::load(pp.d[r], nullptr, Vh, (unsigned)(n.p * 3 * Vh + n.h), 0u, dn);
-            KSIO<CLG_F64>::load(pp.phi[r], nullptr, Vh, (unsigned)(p * 3 * Vh + h), 0u, phix);
-            KSIO<CLG_F64>::load(pp.d[r], nullptr, Vh, (unsigned)(p * 3 * Vh + h), 0u, dx);
-            su3_mv(u, phin, t1);
-            su3_mv(u, dn, t2);
-            // term[3a+c] = t1[a] conj(d(x)[c]) + phi(x)[a] conj(t2[c])   (makeSU3ContractV, SU3.h:505-523)
-            cx term[9];
-            for (int a = 0; a < 3; ++a)
-                for (int c = 0; c < 3; ++c) {
-                    cx acc{0.0, 0.0};
-                    cfmac(acc, dx[c], t1[a]);
-                    cfmac(acc, t2[c], phix[a]);
-                    term[3 * a + c] = acc;
-                }
-            const double f = eta * pp.a[r] * (n.sign < 0 ? -1.0 : 1.0);
-            for (int k = 0; k < 9; ++k) term[k] = cscale(term[k], f);
-            su3_ta(term);
-            for (int k = 0; k < 9; ++k) tot[k] = cadd(tot[k], term[k]);
-        }
-        add_link(F, Vh, el, tot, -1.0);
+    int p, h;
+    const bool valid = order_site(g, tile_y, lane, p, h);
+    if (!valid) {  // idle lanes follow along on a site
+        p = 0;
+        h = 0;
     }
+    const Site s = site_of(g, p, h);
+    Nbr n;
+    int sum = 0;
+    switch (mu) {
+        case 0: n = fwd_nbr<0>(g, s, p); break;
+        case 1: n = fwd_nbr<1>(g, s, p); sum = s.c[0]; break;
+        case 2: n = fwd_nbr<2>(g, s, p); sum = s.c[0] + s.c[1]; break;
+        default: n = fwd_nbr<3>(g, s, p); sum = s.c[0] + s.c[1] + s.c[2]; break;
+    }
+    const unsigned el = (unsigned)((p * 4 + mu) * 9 * Vh + h);
+    const unsigned en = (unsigned)(n.p * 3 * Vh + n.h), ex = (unsigned)(p * 3 * Vh + h);
+    cx m1[9], m2[9], mine[3] = {};
+#pragma unroll
+    for (int k = 0; k < 9; ++k) m1[k] = m2[k] = cx{0.0, 0.0};
+    // wave w brings vector w & 1 of pole r + w / 2
+    auto fetch = [&](int r) {
+        const int rr = r + (mu >> 1);
+        if (rr >= npole) return;
+        KSIO<CLG_F64>::load((mu & 1) ? pp.d[rr] : pp.phi[rr], nullptr, Vh, ex, 0u, mine);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) mine[c] = cscale(mine[c], pp.a[rr]);
+    };
+    fetch(0);
+    for (int r = 0, buf = 0; r < npole; r += 2, buf ^= 1) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) own[buf][mu][c][lane] = make_double2(mine[c].x, mine[c].y);
+        cx phin[2][3], dn[2][3];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            if (i > 0 && r + i >= npole) continue;
+            KSIO<CLG_F64>::load(pp.phi[r + i], nullptr, Vh, en, 0u, phin[i]);
+            KSIO<CLG_F64>::load(pp.d[r + i], nullptr, Vh, en, 0u, dn[i]);
+        }
+        if (r + 2 < npole) fetch(r + 2);
+        __syncthreads();  // one a round: the next one writes the other buffer
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            if (r + i < npole) {
+                cx phix[3], dx[3];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    const double2 v = own[buf][2 * i][c][lane], w = own[buf][2 * i + 1][c][lane];
+                    phix[c] = cx{v.x, v.y};
+                    dx[c] = cx{w.x, w.y};
+                }
+                outer_add(phin[i], dx, m1);
+                outer_add(phix, dn[i], m2);
+            }
+        }
+    }
+    if (!valid) return;
+    cx u[9], f[9];
+    LinkIO<CLG_F64, 18>::load<true>(U, Vh, el, u);
+    su3_mm(u, m1, f);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) cfmac(f[3 * i + j], u[3 * j + k], m2[3 * i + k]);  // += M2 U^dagger
+    su3_ta(f);
+    add_link(F, Vh, el, f, ((sum & 1) != 0) == (n.sign < 0) ? -1.0 : 1.0);  // F -= eta sign f
 }
 
 int check_force_args(const clg_field_s* force, const clg_field_s* gauge) {
@@ -182,9 +212,9 @@ int clg_wilson_force_kernel(clg_context ctx, clg_field force, clg_field gauge, c
                   "need FULL FP64 Wilson fields");
     Geo g = make_geo(inv_dddag);
     (void)hipSetDevice(ctx->device);
-    k_wilson_force<<<sched_grid(g.Vh, 2, kForceBlock, 8, 1), kForceBlock, 0, ctx->stream>>>(g, (const char*)inv_dddag->data,
-                                                                       (const char*)inv_d->data,
-                                                                       (const char*)gauge->data, (char*)force->data, kappa);
+    const SiteOrder o = site_order(g);
+    k_wilson_force<<<o.grid, 256, 0, ctx->stream>>>(g, (const char*)inv_dddag->data, (const char*)inv_d->data,
+                                                     (const char*)gauge->data, (char*)force->data, kappa, o.tile_y);
     CLG_HIP(hipGetLastError());
     return CLG_OK;
 }
@@ -207,8 +237,8 @@ int clg_ks_force_kernel(clg_context ctx, clg_field force, clg_field gauge, const
     }
     Geo g = make_geo(phis[0]);
     (void)hipSetDevice(ctx->device);
-    k_ks_force<<<sched_grid(g.Vh, 2, kForceBlock, 8, 1), kForceBlock, 0, ctx->stream>>>(g, pp, npole, (const char*)gauge->data,
-                                                                   (char*)force->data);
+    const SiteOrder o = site_order(g);
+    k_ks_force<<<o.grid, 256, 0, ctx->stream>>>(g, pp, npole, (const char*)gauge->data, (char*)force->data, o.tile_y);
     CLG_HIP(hipGetLastError());
     return CLG_OK;
 }

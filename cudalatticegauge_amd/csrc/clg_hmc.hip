@@ -81,21 +81,6 @@ __device__ __forceinline__ PH at_step(const Site& s, int p, Step a) { return PH{
 __device__ __forceinline__ PH at_steps(const Site& s, int p, Step a, Step b) {
     return PH{p ^ a.flip ^ b.flip, (s.lex + a.dlex + b.dlex) >> 1};
 }
-// work order of the site kernels in 64-site blocks: the tiled plane order where it keeps the lanes busy
-// (neighbour planes then meet in one XCD's L2), else XCD slabs.  Gauge force at 32^3x16: eight tiles along y
-// 322 us, 2 x 4 tiles 341, 4 x 2 tiles 346, slabs 344; at 21x19x25x18, where a plane fills 4 of 3.5 blocks,
-// all within 1 %.
-struct SiteOrder {
-    int tile_y;  // 0: slabs
-    unsigned grid;
-};
-SiteOrder site_order(const Geo& g) {
-    if (tile64_fits(g, 8)) return SiteOrder{8, tile64_grid(g, 2, 8)};
-    return SiteOrder{0, sched_grid(g.Vh, 2, 64, 8, 1)};
-}
-__device__ __forceinline__ bool order_site(const Geo& g, int tile_y, int lane, int& p, int& h) {
-    return tile_y ? tile64_site(g, 2, 0, tile_y, 0, lane, p, h) : block_site(logical_wg(8), 64, (unsigned)lane, g.Vh, 2, 0, 1, p, h);
-}
 __device__ __forceinline__ void load_link(const char* U, const Geo& g, PH s, int mu, cd* m) {
     LinkIO<CLG_F64, 18>::load(U, g.Vh, (unsigned)((s.p * 4 + mu) * 9 * g.Vh + s.h), m);
 }

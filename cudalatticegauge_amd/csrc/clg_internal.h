@@ -230,6 +230,18 @@ inline bool tile64_fits(const Geo& g, int TY) {
     return 8L * g.Vh >= 7L * lanes;
 }
 
+// work order of the site kernels in 64-site blocks: the tiled plane order where it keeps the lanes busy
+// (neighbour planes then meet in one XCD's L2), else XCD slabs.  Gauge force at 32^3x16: eight tiles along y
+// 322 us, 2 x 4 tiles 341, 4 x 2 tiles 346, slabs 344; at 21x19x25x18, where a plane fills 4 of 3.5 blocks,
+// all within 1 %.
+struct SiteOrder {
+    int tile_y;  // 0: slabs
+    unsigned grid;
+};
+inline SiteOrder site_order(const Geo& g) {
+    if (tile64_fits(g, 8)) return SiteOrder{8, tile64_grid(g, 2, 8)};
+    return SiteOrder{0, sched_grid(g.Vh, 2, 64, 8, 1)};
+}
 }  // namespace clg
 
 // ======================================================================= device side
@@ -413,6 +425,10 @@ __device__ __forceinline__ bool tile64_site(const clg::Geo& g, int nblk, int pba
     const int x = x0 + (ymajor ? minor : major), y = y0 + (ymajor ? major : minor);
     h = (x * g.L[1] + y) * plane + sub * 64 + lane;
     return sub * 64 + lane < plane;
+}
+// site of a full-lattice launch in clg::site_order
+__device__ __forceinline__ bool order_site(const clg::Geo& g, int tile_y, int lane, int& p, int& h) {
+    return tile_y ? tile64_site(g, 2, 0, tile_y, 0, lane, p, h) : block_site(logical_wg(8), 64, (unsigned)lane, g.Vh, 2, 0, 1, p, h);
 }
 __device__ __forceinline__ bool map_site(int Vh, int nblk, int pbase, int xcd, int pinter, int& p, int& h) {
     return block_site(logical_wg(xcd), Vh, nblk, pbase, pinter, p, h);
