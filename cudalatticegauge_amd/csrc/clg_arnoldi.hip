@@ -84,13 +84,8 @@ __global__ __launch_bounds__(kArnBlock) void k_arn_dots(long n, ArnPtrs<P> V, in
         }
     }
     __shared__ double sm[kArnBlock / 64][kArnRows];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-    for (int r = 0; r < kArnRows; ++r) v[r] = wave_sum(v[r]);
-    if (lane == 0) {
-#pragma unroll
-        for (int r = 0; r < kArnRows; ++r) sm[wv][r] = v[r];
-    }
+    const int wv = threadIdx.x >> 6;
+    wave_fold<kArnRows>(v, sm[wv]);
     __syncthreads();
     const int G = (int)gridDim.x;
     for (int r = threadIdx.x; r < kArnRows; r += blockDim.x) {
@@ -296,7 +291,7 @@ __global__ __launch_bounds__(kArnBlock) void k_arn_subfuse(long n, ArnPtrs<P> V,
         }
     }
     __shared__ double sm[kArnBlock / 64][kArnRows];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int wv = threadIdx.x >> 6;
     const int G = (int)gridDim.x, nch = (nv + kArnK - 1) / kArnK;
     for (int c = 0; c < nch; ++c) {
         const int k0 = c * kArnK, kk = min(kArnK, nv - k0);
@@ -329,13 +324,8 @@ __global__ __launch_bounds__(kArnBlock) void k_arn_subfuse(long n, ArnPtrs<P> V,
                 }
             }
         }
-#pragma unroll
-        for (int t = 0; t < kArnRows; ++t) a[t] = wave_sum(a[t]);
         if (c > 0) __syncthreads();  // the previous chunk's sums have been read
-        if (lane == 0) {
-#pragma unroll
-            for (int t = 0; t < kArnRows; ++t) sm[wv][t] = a[t];
-        }
+        wave_fold<kArnRows>(a, sm[wv]);
         __syncthreads();
         for (int t = threadIdx.x; t < kArnRows; t += blockDim.x) {
             double s = 0.0;

@@ -647,32 +647,19 @@ __global__ __launch_bounds__(kRedBlock) void k_bmultiaxpy(const BTab* T, Act act
 // nblk partials (nr values each) in a fixed order; totals r < nout go to out[s*stride + r], the one
 // after them to out2[s*stride]; flag (nullable) gets total_0 < eta * ref[s*stride].  Systems with
 // cond[s*stride] == 0 are skipped, as in the first stage.
-__global__ __launch_bounds__(kRedBlock) void k_bred_finish(Act act, const double* __restrict__ partial, int nblk,
+__global__ __launch_bounds__(kFinBlock) void k_bred_finish(Act act, const double* __restrict__ partial, int nblk,
                                                            int nr, double* out, int nout, double* out2,
                                                            const double* cond, const double* ref, double eta,
                                                            double* flag, int stride) {
     const int s = act.idx[blockIdx.y];
     if (cond && cond[(size_t)s * stride] == 0.0) return;
-    const double* pp = partial + (size_t)blockIdx.y * nblk * nr;
-    __shared__ double sm[kRedBlock / 64][2 * kMaxM + 1];
-    __shared__ double tot[2 * kMaxM + 1];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (int r = 0; r < nr; ++r) {
-        double a = 0;
-        for (int b = threadIdx.x; b < nblk; b += blockDim.x) a += pp[(size_t)b * nr + r];
-        a = wave_sum(a);
-        if (lane == 0) sm[wv][r] = a;
-    }
-    __syncthreads();
+    __shared__ double tot[kFinMax];
+    partial_totals<kFinBlock>(partial + (size_t)blockIdx.y * nblk * nr, nblk, nr, tot);
     if ((int)threadIdx.x < nr) {
         const int r = threadIdx.x;
-        double t = 0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += sm[w][r];
-        tot[r] = t;
-        if (r < nout) out[(size_t)s * stride + r] = t;
-        else if (out2) out2[(size_t)s * stride] = t;
+        if (r < nout) out[(size_t)s * stride + r] = tot[r];
+        else if (out2) out2[(size_t)s * stride] = tot[r];
     }
-    __syncthreads();
     if (flag && threadIdx.x == 0) flag[(size_t)s * stride] = tot[0] < eta * ref[(size_t)s * stride] ? 1.0 : 0.0;
 }
 
@@ -751,42 +738,11 @@ __global__ void k_bhess_update(double* ws, size_t stride, size_t offH, size_t of
 
 // Givens QR of the (m+1) x m Hessenberg with g = |r| e1 and back substitution (RotateH / SolveY,
 // CSolverGMRES.cpp:262-358) for each system, FP64
-__global__ void k_bgmres_lsq(double* ws, size_t stride, WsLayout L, Act act) {
-    if (threadIdx.x != 0) return;
-    const int s = act.idx[blockIdx.y];
-    double* base = ws + (size_t)s * stride;
-    typedef C2<double> c;
-    const int ld = L.ld, m = L.m;
-    double* H = base + L.offH;
-    auto Hp = [&](int r, int col) -> c* { return reinterpret_cast<c*>(H + 2 * (col * ld + r)); };
-    c* G = reinterpret_cast<c*>(base + L.offG);
-    c* Y = reinterpret_cast<c*>(base + L.offY);
+__global__ __launch_bounds__(64) void k_bgmres_lsq(double* ws, size_t stride, WsLayout L, Act act) {
+    __shared__ cd sm[kMaxM * (kMaxM + 1)];
+    double* base = ws + (size_t)act.idx[blockIdx.y] * stride;
     double* sc = base + L.offS;
-    G[0] = c{sqrt(sc[0]), 0.0};
-    for (int k = 1; k <= m; ++k) G[k] = c{0.0, 0.0};
-    for (int k = 0; k < m; ++k) {
-        const c hkk = *Hp(k, k), hk1 = *Hp(k + 1, k);
-        const double den = 1.0 / sqrt(hkk.x * hkk.x + hkk.y * hkk.y + hk1.x * hk1.x + hk1.y * hk1.y);
-        const c cs = cscale(hkk, den), sn = cscale(hk1, den);
-        const c csh = cconj(cs), snh = cconj(sn);
-        for (int jj = k; jj < m; ++jj) {
-            const c hkj = *Hp(k, jj), h1j = *Hp(k + 1, jj);
-            *Hp(k, jj) = cadd(cmul(csh, hkj), cmul(snh, h1j));
-            *Hp(k + 1, jj) = csub(cmul(cs, h1j), cmul(sn, hkj));
-        }
-        const c mg = c{-G[k].x, -G[k].y};
-        G[k] = cmul(csh, G[k]);
-        G[k + 1] = cmul(sn, mg);
-    }
-    sc[2] = G[m].x * G[m].x + G[m].y * G[m].y;
-    sc[3] = sqrt(sc[2]);
-    for (int k = m - 1; k >= 0; --k) {
-        c acc = G[k];
-        for (int jj = k + 1; jj < m; ++jj) acc = csub(acc, cmul(*Hp(k, jj), Y[jj]));
-        const c d = *Hp(k, k);
-        const double dd = d.x * d.x + d.y * d.y;
-        Y[k] = c{(acc.x * d.x + acc.y * d.y) / dd, (acc.y * d.x - acc.x * d.y) / dd};
-    }
+    gmres_lsq_wave(base + L.offH, L.ld, L.m, sc[0], base + L.offY, sc + 2, sm);
 }
 
 // ---- batched BLAS on FP16-storage vectors (one parity block each; see clg_blas16.hip for the
@@ -1024,7 +980,7 @@ __global__ __launch_bounds__(kRedBlock) void k_bh_gs_project(const BTab* T, Act 
 // K = 1 - A (the batched inner solve): H(i, j) = delta_ij - (h_i + flag c2_i), H(j+1, j) = -|w''|.
 // gs (per system, 36 doubles): [0] |w|^2 (in), [1] |w''|^2, [2] 1/|w''|, [3] flag, [4..) c2.
 template <int K>
-__global__ __launch_bounds__(kRedBlock) void k_bgs_finish(Act act, const double* __restrict__ partial, int nblk,
+__global__ __launch_bounds__(kFinBlock) void k_bgs_finish(Act act, const double* __restrict__ partial, int nblk,
                                                            double* ws, int stride, int offh, int offgs, int fast_ok) {
     constexpr int NR = 2 * K + 1;
     const int s = act.idx[blockIdx.y];
@@ -1045,29 +1001,8 @@ __global__ __launch_bounds__(kRedBlock) void k_bgs_finish(Act act, const double*
         }
         return;
     }
-    __shared__ double sm[kRedBlock / 64][NR];
-    __shared__ double tot[NR];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    double acc[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) acc[r] = 0;
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) acc[r] += pp[(size_t)b * NR + r];
-    }
-#pragma unroll
-    for (int r = 0; r < NR; ++r) acc[r] = wave_sum(acc[r]);
-    if (lane == 0) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) sm[wv][r] = acc[r];
-    }
-    __syncthreads();
-    if (threadIdx.x < NR) {
-        double t = 0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += sm[w][threadIdx.x];
-        tot[threadIdx.x] = t;
-    }
-    __syncthreads();
+    __shared__ double tot[kFinMax];
+    partial_totals<kFinBlock>(pp, nblk, NR, tot);
     const double w2 = tot[2 * K];
     const bool flag = w2 < 0.5 * gs[0];
     const int i = threadIdx.x;
@@ -1337,7 +1272,7 @@ struct BatchSolver {
             k_bmultidot<P, K, false><<<grid, kRedBlock, 0, ctx->stream>>>(dtab, A, m, ctx->red_partial, cond,
                                                                           (int)L.stride);
         CLG_HIP(hipGetLastError());
-        k_bred_finish<<<dim3(1, A.n), kRedBlock, 0, ctx->stream>>>(A, ctx->red_partial, (int)g, 2 * K + (wn ? 1 : 0),
+        k_bred_finish<<<dim3(1, A.n), kFinBlock, 0, ctx->stream>>>(A, ctx->red_partial, (int)g, 2 * K + (wn ? 1 : 0),
                                                                    out_base + ostride_off, 2 * K, wn, cond, nullptr,
                                                                    0.0, nullptr, (int)L.stride);
         CLG_HIP(hipGetLastError());
@@ -1356,7 +1291,7 @@ struct BatchSolver {
                                                                            ctx->red_partial, cond);
         CLG_HIP(hipGetLastError());
         if (nrm) {
-            k_bred_finish<<<dim3(1, A.n), kRedBlock, 0, ctx->stream>>>(A, ctx->red_partial, (int)g, 1, nrm, 1, nullptr,
+            k_bred_finish<<<dim3(1, A.n), kFinBlock, 0, ctx->stream>>>(A, ctx->red_partial, (int)g, 1, nrm, 1, nullptr,
                                                                        cond, ref, eta, flag, (int)L.stride);
             CLG_HIP(hipGetLastError());
         }
@@ -1428,7 +1363,7 @@ struct BatchSolver {
             }
             CLG_HIP(hipGetLastError());
             k_bnorm2<P><<<rgrid, kRedBlock, 0, ctx->stream>>>(dtab, A, 0, ctx->red_partial);
-            k_bred_finish<<<dim3(1, A.n), kRedBlock, 0, ctx->stream>>>(A, ctx->red_partial, (int)rg, 1, ws + L.offS, 1,
+            k_bred_finish<<<dim3(1, A.n), kFinBlock, 0, ctx->stream>>>(A, ctx->red_partial, (int)rg, 1, ws + L.offS, 1,
                                                                        nullptr, nullptr, nullptr, 0.0, nullptr,
                                                                        (int)L.stride);
             k_bscale<P><<<egrid, 256, 0, ctx->stream>>>(dtab, A, 0, 0, ws + L.offS, (int)L.stride);
@@ -1500,7 +1435,7 @@ struct BatchSolver {
             }
             CLG_HIP(hipGetLastError());
             k_bh_norm2<<<rgrid, kRedBlock, 0, ctx->stream>>>(dtab, A, 0, ctx->red_partial);
-            k_bred_finish<<<dim3(1, A.n), kRedBlock, 0, ctx->stream>>>(A, ctx->red_partial, (int)rg, 1, ws + L.offS, 1,
+            k_bred_finish<<<dim3(1, A.n), kFinBlock, 0, ctx->stream>>>(A, ctx->red_partial, (int)rg, 1, ws + L.offS, 1,
                                                                        nullptr, nullptr, nullptr, 0.0, nullptr, stride);
             k_bh_scale<<<egrid, 256, 0, ctx->stream>>>(dtab, A, 0, 0, ws + L.offS, stride);
             CLG_HIP(hipGetLastError());
@@ -1514,12 +1449,12 @@ struct BatchSolver {
                 const int nv = j + 1;
 #define CALL(KK)                                                                                                 \
     k_bh_multidot<KK><<<rgrid, kRedBlock, 0, ctx->stream>>>(dtab, A, m, ctx->red_partial);                       \
-    k_bred_finish<<<dim3(1, A.n), kRedBlock, 0, ctx->stream>>>(A, ctx->red_partial, (int)rg, 2 * KK + 1,         \
+    k_bred_finish<<<dim3(1, A.n), kFinBlock, 0, ctx->stream>>>(A, ctx->red_partial, (int)rg, 2 * KK + 1,         \
                                                                ws + offh, 2 * KK, ws + L.offGS, nullptr, nullptr, \
                                                                0.0, nullptr, stride);                            \
     k_bh_gs_project<KK><<<rgrid, kRedBlock, 0, ctx->stream>>>(dtab, A, m, j < m - 1 ? j + 1 : m, ws, stride, offh, \
                                                               ctx->red_partial, (int)L.offGS, j < m - 1 ? 1 : 0); \
-    k_bgs_finish<KK><<<dim3(1, A.n), kRedBlock, 0, ctx->stream>>>(A, ctx->red_partial, (int)rg, ws, stride, offh, \
+    k_bgs_finish<KK><<<dim3(1, A.n), kFinBlock, 0, ctx->stream>>>(A, ctx->red_partial, (int)rg, ws, stride, offh, \
                                                                   (int)L.offGS, j < m - 1 ? 1 : 0);              \
     if (j < m - 1)                                                                                               \
         k_bh_gs_finalize<KK><<<egrid, 256, 0, ctx->stream>>>(dtab, A, j + 1, ws, stride, (int)L.offGS);

@@ -300,32 +300,16 @@ __global__ __launch_bounds__(kRedBlock) void k_multiaxpy_ch(long n, PtrsN<P> V, 
 }
 // finish of k_multidot_ch: one workgroup per chunk (blockIdx.y); chunk c writes its 2*kk sums to
 // out[2*kMaxK*c ..], chunk 0 also |w|^2 to wn (nullable)
-__global__ __launch_bounds__(kRedBlock) void k_red_finish_ch(const double* __restrict__ partial, int nblk, int nv,
+__global__ __launch_bounds__(kFinBlock) void k_red_finish_ch(const double* __restrict__ partial, int nblk, int nv,
                                                              double* out, double* wn, const int* cond) {
     constexpr int NR = 2 * kMaxK + 1;
     if (cond && *cond == 0) return;
     const int ch = (int)blockIdx.y, kk = min(kMaxK, nv - ch * kMaxK);
-    const double* pp = partial + (size_t)ch * nblk * NR;
-    __shared__ double sm[kRedBlock / 64][NR];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    double acc[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) acc[r] = 0;
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) acc[r] += pp[(size_t)b * NR + r];
-    }
-#pragma unroll
-    for (int r = 0; r < NR; ++r) acc[r] = wave_sum(acc[r]);
-    if (lane == 0) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) sm[wv][r] = acc[r];
-    }
-    __syncthreads();
+    __shared__ double tot[kFinMax];
+    partial_totals<kFinBlock>(partial + (size_t)ch * nblk * NR, nblk, NR, tot);
     if (threadIdx.x < NR) {
         const int r = threadIdx.x;
-        double t = 0;
-        for (int q = 0; q < (int)(blockDim.x >> 6); ++q) t += sm[q][r];
+        const double t = tot[r];
         if (r < 2 * kk) out[2 * kMaxK * ch + r] = t;
         else if (r == NR - 1 && ch == 0 && wn) wn[0] = t;
     }
@@ -336,40 +320,18 @@ __global__ __launch_bounds__(kRedBlock) void k_red_finish_ch(const double* __res
 // out2[0] (when given).  flag (nullable): *flag = (total_0 < eta * ref[0]).  cond (nullable): skip
 // when *cond == 0, as the first stage did.  Every load of a thread is independent (block-major
 // sweep with NR accumulators), so they all stay in flight.
-template <int NR>
-__global__ __launch_bounds__(kRedBlock) void k_red_finish(const double* __restrict__ partial, int nblk, double* out,
+__global__ __launch_bounds__(kFinBlock) void k_red_finish(const double* __restrict__ partial, int nblk, int nr, double* out,
                                                           int nout, double* out2, const int* cond, const double* ref,
                                                           double eta, int* flag) {
     if (cond && *cond == 0) return;
-    __shared__ double sm[kRedBlock / 64][NR];
-    __shared__ double tot[NR];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    double acc[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) acc[r] = 0;
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) acc[r] += partial[(size_t)b * NR + r];
-    }
-#pragma unroll
-    for (int r = 0; r < NR; ++r) acc[r] = wave_sum(acc[r]);
-    if (lane == 0) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) sm[wv][r] = acc[r];
-    }
-    __syncthreads();
-    if (threadIdx.x < NR) {
+    __shared__ double tot[kFinMax];
+    partial_totals<kFinBlock>(partial, nblk, nr, tot);
+    if ((int)threadIdx.x < nr) {
         const int r = threadIdx.x;
-        double t = 0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += sm[w][r];
-        tot[r] = t;
-        if (r < nout) out[r] = t;
-        else if (out2) out2[r - nout] = t;
+        if (r < nout) out[r] = tot[r];
+        else if (out2) out2[r - nout] = tot[r];
     }
-    if (flag) {
-        __syncthreads();
-        if (threadIdx.x == 0) *flag = tot[0] < eta * ref[0] ? 1 : 0;
-    }
+    if (flag && threadIdx.x == 0) *flag = tot[0] < eta * ref[0] ? 1 : 0;
 }
 
 // out_i = sum_{j<X} in_j M[j*Y + i] (i < Y <= YM) for FP64 complex vectors of n elements, M in
@@ -410,6 +372,55 @@ __global__ __launch_bounds__(256) void k_vmm(VmmArgs a, const double* __restrict
     }
 }
 
+// ---- Hessenberg column of one Gram-Schmidt step (one workgroup); the fast form's and the general one's
+// the column of the fast form from the projections h
+template <int K>
+__device__ __forceinline__ void gs_fast_column(const double* h, double w2, double* hcol, int j, int shifted) {
+    const int i = threadIdx.x;
+    if (i < K) {
+        hcol[2 * i] = shifted ? (i == j ? 1.0 : 0.0) - h[2 * i] : h[2 * i];
+        hcol[2 * i + 1] = shifted ? -h[2 * i + 1] : h[2 * i + 1];
+    }
+    if (i == 0) {
+        const double f = sqrt(w2);
+        hcol[2 * (j + 1)] = shifted ? -f : f;
+        hcol[2 * (j + 1) + 1] = 0.0;
+    }
+}
+// the column from h (hcol) and the second-pass totals
+template <int K>
+__device__ __forceinline__ void gs_slow_column(const double* tot, double* hcol, int j, int shifted, double* sc) {
+    const double w2 = tot[2 * K];
+    const bool flag = w2 < 0.5 * sc[0];
+    const int i = threadIdx.x;
+    if (i < K) {
+        double re = hcol[2 * i], im = hcol[2 * i + 1];
+        if (flag) {
+            re += tot[2 * i];
+            im += tot[2 * i + 1];
+        }
+        if (shifted) {
+            re = (i == j ? 1.0 : 0.0) - re;
+            im = -im;
+        }
+        hcol[2 * i] = re;
+        hcol[2 * i + 1] = im;
+        sc[4 + 2 * i] = tot[2 * i];
+        sc[4 + 2 * i + 1] = tot[2 * i + 1];
+    }
+    if (i == 0) {
+        double c2 = 0;
+        for (int k = 0; k < 2 * K; ++k) c2 += tot[k] * tot[k];
+        double f2 = flag ? w2 - c2 : w2;
+        if (!(f2 > 1e-300)) f2 = 1e-300;
+        const double f = sqrt(f2);
+        hcol[2 * (j + 1)] = shifted ? -f : f;
+        hcol[2 * (j + 1) + 1] = 0.0;
+        sc[1] = f2;
+        sc[2] = 1.0 / f;
+        sc[3] = flag ? 1.0 : 0.0;
+    }
+}
 // ---- fused Gram-Schmidt step of the Arnoldi process (see blas_gs_step)
 // w' = w - sum_k h_k V_k (h = the first-pass projections, on device) is stored, and the same pass
 // yields the partials of V_k^H w' (2K values) and |w'|^2 (the last one).
@@ -417,16 +428,29 @@ __global__ __launch_bounds__(256) void k_vmm(VmmArgs a, const double* __restrict
 // When that keeps at least half of |w|^2 (no second pass will be needed), the step's fast form
 // applies: w' / |w'| goes straight to vnext and no partials are taken.  Workgroup 0 records the choice
 // in sc ([1] |w'|^2, [2] 1/|w'|, [3] 2 for the fast form, else 0) for the finish and finalize.
-template <int P, int K>
-__global__ __launch_bounds__(kRedBlock) void k_gs_project(long n, Ptrs<P> V, const double* __restrict__ h,
-                                                           typename Pk<P>::T* w, double* partial, double* sc,
-                                                           typename Pk<P>::T* vnext) {
+// MERGED (small vectors): h and |w|^2 are not finished yet; every workgroup totals the projection pass's nin
+// partials itself (two launches less per step), workgroup 0 stores h to hcol and |w|^2 to sc[0], and in the fast
+// form also the finished column.
+template <int P, int K, bool MERGED>
+__global__ __launch_bounds__(kRedBlock) void k_gs_project(long n, Ptrs<P> V, double* hcol, typename Pk<P>::T* w, double* partial,
+                                                           double* sc, typename Pk<P>::T* vnext,
+                                                           const double* __restrict__ pin, int nin, int j, int shifted) {
     constexpr int NC = Pk<P>::NC;
+    __shared__ double tot[MERGED ? kFinMax : 1];
+    const double* h = hcol;
+    if constexpr (MERGED) {
+        partial_totals<kRedBlock>(pin, nin, 2 * K + 1, tot);
+        h = tot;
+        if (blockIdx.x == 0) {
+            if (threadIdx.x < 2 * K) hcol[threadIdx.x] = tot[threadIdx.x];
+            else if (threadIdx.x == 2 * K) sc[0] = tot[2 * K];
+        }
+    }
     double hr[K], hi[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) { hr[k] = h[2 * k]; hi[k] = h[2 * k + 1]; }
     if (vnext) {
-        const double w2 = sc[0];
+        const double w2 = MERGED ? tot[2 * K] : sc[0];
         double b2 = w2;
 #pragma unroll
         for (int k = 0; k < K; ++k) b2 -= hr[k] * hr[k] + hi[k] * hi[k];
@@ -438,6 +462,8 @@ __global__ __launch_bounds__(kRedBlock) void k_gs_project(long n, Ptrs<P> V, con
                 sc[2] = 1.0 / sqrt(b2);
             }
         }
+        if constexpr (MERGED)
+            if (fast && blockIdx.x == 0) gs_fast_column<K>(tot, b2, hcol, j, shifted);
         if (fast) {
             const double inv = 1.0 / sqrt(b2);
             GRID_STRIDE(i, n) {
@@ -509,90 +535,50 @@ __global__ __launch_bounds__(kRedBlock) void k_gs_project(long n, Ptrs<P> V, con
 // (V orthonormal), H(j+1, j) = +-|w''|.  sc: [0] |w|^2 (in), [1] |w''|^2, [2] 1/|w''|, [3] flag,
 // [4..4+2K) c2.
 template <int K>
-__global__ __launch_bounds__(kRedBlock) void k_gs_finish(const double* __restrict__ partial, int nblk, double* hcol,
+__global__ __launch_bounds__(kFinBlock) void k_gs_finish(const double* __restrict__ partial, int nblk, double* hcol,
                                                           int j, int shifted, double* sc, int fast_ok) {
     constexpr int NR = 2 * K + 1;
-    if (fast_ok && sc[3] == 2.0) {
-        // the projection pass took the fast form: H(i, j) = h_i, H(j+1, j) = |w'| from sc
-        const int i = threadIdx.x;
-        if (i < K && shifted) {
-            hcol[2 * i] = (i == j ? 1.0 : 0.0) - hcol[2 * i];
-            hcol[2 * i + 1] = -hcol[2 * i + 1];
-        }
-        if (i == 0) {
-            const double f = sqrt(sc[1]);
-            hcol[2 * (j + 1)] = shifted ? -f : f;
-            hcol[2 * (j + 1) + 1] = 0.0;
-        }
+    if (fast_ok && sc[3] == 2.0) {  // the projection pass took the fast form: h in hcol, |w'|^2 in sc
+        gs_fast_column<K>(hcol, sc[1], hcol, j, shifted);
         return;
     }
-    __shared__ double sm[kRedBlock / 64][NR];
-    __shared__ double tot[NR];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    double acc[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) acc[r] = 0;
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) acc[r] += partial[(size_t)b * NR + r];
-    }
-#pragma unroll
-    for (int r = 0; r < NR; ++r) acc[r] = wave_sum(acc[r]);
-    if (lane == 0) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) sm[wv][r] = acc[r];
-    }
-    __syncthreads();
-    if (threadIdx.x < NR) {
-        double t = 0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += sm[w][threadIdx.x];
-        tot[threadIdx.x] = t;
-    }
-    __syncthreads();
-    const double w2 = tot[2 * K];
-    const bool flag = w2 < 0.5 * sc[0];
-    const int i = threadIdx.x;
-    if (i < K) {
-        double re = hcol[2 * i], im = hcol[2 * i + 1];
-        if (flag) {
-            re += tot[2 * i];
-            im += tot[2 * i + 1];
-        }
-        if (shifted) {
-            re = (i == j ? 1.0 : 0.0) - re;
-            im = -im;
-        }
-        hcol[2 * i] = re;
-        hcol[2 * i + 1] = im;
-        sc[4 + 2 * i] = tot[2 * i];
-        sc[4 + 2 * i + 1] = tot[2 * i + 1];
-    }
-    if (i == 0) {
-        double c2 = 0;
-        for (int k = 0; k < 2 * K; ++k) c2 += tot[k] * tot[k];
-        double f2 = flag ? w2 - c2 : w2;
-        if (!(f2 > 1e-300)) f2 = 1e-300;
-        const double f = sqrt(f2);
-        hcol[2 * (j + 1)] = shifted ? -f : f;
-        hcol[2 * (j + 1) + 1] = 0.0;
-        sc[1] = f2;
-        sc[2] = 1.0 / f;
-        sc[3] = flag ? 1.0 : 0.0;
-    }
+    __shared__ double tot[kFinMax];
+    partial_totals<kFinBlock>(partial, nblk, NR, tot);
+    gs_slow_column<K>(tot, hcol, j, shifted, sc);
 }
 
 // vnext = (w' - flag sum_k c2_k V_k) / |w''| with flag, c2 and 1/|w''| from k_gs_finish
-template <int P, int K>
+// MERGED (small vectors): k_gs_finish has not run; when the fast form was not taken every workgroup totals the
+// projection pass's nin partials, and workgroup 0 writes the column and sc.
+template <int P, int K, bool MERGED>
 __global__ __launch_bounds__(kRedBlock) void k_gs_finalize(long n, Ptrs<P> V, const typename Pk<P>::T* __restrict__ w,
-                                                            typename Pk<P>::T* vnext, const double* __restrict__ sc) {
+                                                            typename Pk<P>::T* vnext, double* sc,
+                                                            const double* __restrict__ pin, int nin, double* hcol, int j,
+                                                            int shifted) {
     constexpr int NC = Pk<P>::NC;
     if (sc[3] == 2.0) return;  // the projection pass wrote vnext (fast form)
-    const bool flag = sc[3] != 0.0;
-    const double inv = sc[2];
+    __shared__ double tot[MERGED ? kFinMax : 1];
+    const double* c2 = sc + 4;
+    bool flag;
+    double inv;
+    if constexpr (MERGED) {
+        partial_totals<kRedBlock>(pin, nin, 2 * K + 1, tot);
+        c2 = tot;
+        const double w2 = tot[2 * K];
+        flag = w2 < 0.5 * sc[0];
+        double f2 = w2;
+        if (flag)
+            for (int k = 0; k < 2 * K; ++k) f2 -= tot[k] * tot[k];
+        inv = 1.0 / sqrt(f2 > 1e-300 ? f2 : 1e-300);
+        if (blockIdx.x == 0) gs_slow_column<K>(tot, hcol, j, shifted, sc);
+    } else {
+        flag = sc[3] != 0.0;
+        inv = sc[2];
+    }
     if (flag) {
         double cr[K], ci[K];
 #pragma unroll
-        for (int k = 0; k < K; ++k) { cr[k] = sc[4 + 2 * k]; ci[k] = sc[4 + 2 * k + 1]; }
+        for (int k = 0; k < K; ++k) { cr[k] = c2[2 * k]; ci[k] = c2[2 * k + 1]; }
         GRID_STRIDE(i, n) {
             typename Pk<P>::T raw[K];
 #pragma unroll
@@ -624,10 +610,13 @@ __global__ __launch_bounds__(kRedBlock) void k_gs_finalize(long n, Ptrs<P> V, co
     }
 }
 
+// workgroups of a reduction: four packets a lane, but one a lane while that gives at most kMergeGrid workgroups (a
+// small vector's pass is a chain of latencies: 12-vector multi-dot at 8^4 7.9 -> 4.4 us)
+constexpr long kMergeGrid = 256;
 unsigned red_grid(clg_context ctx, long n) {
-    long g = (n + kRedBlock * 4 - 1) / (kRedBlock * 4);
+    const long one = (n + kRedBlock - 1) / kRedBlock, four = (one + 3) / 4;
     const long cap = std::min<long>(kMaxRedGrid, (long)ctx->num_cu * 4);
-    return (unsigned)std::max<long>(1, std::min(g, cap));
+    return (unsigned)std::max<long>(1, std::max(std::min(one, kMergeGrid), std::min(four, cap)));
 }
 unsigned ew_grid(clg_context ctx, long n) {
     long g = (n + 255) / 256;
@@ -784,16 +773,8 @@ int blas_conj(clg_context ctx, clg_field_s* dst, const clg_field_s* src) {
 // second stage of a reduction whose first stage wrote nblk x nr partials to `partial`
 static int red_finish_at(clg_context ctx, const double* partial, unsigned nblk, int nr, double* out, int nout,
                          double* out2, const int* cond, const double* ref, double eta, int* flag) {
-#define FIN(N)                                                                                                    \
-    case N:                                                                                                       \
-        k_red_finish<N><<<1, kRedBlock, 0, ctx->stream>>>(partial, (int)nblk, out, nout, out2, cond, ref, eta, flag); \
-        break;
-    switch (nr) {
-        FIN(1) FIN(2) FIN(3) FIN(5) FIN(7) FIN(9) FIN(11) FIN(13) FIN(15) FIN(17) FIN(19) FIN(21) FIN(23) FIN(25)
-        FIN(27) FIN(29) FIN(31) FIN(33)
-        default: CLG_CHECK_ARG(false, "no reduction finish for %d values", nr);
-    }
-#undef FIN
+    CLG_CHECK_ARG(nr >= 1 && nr <= kFinMax, "no reduction finish for %d values", nr);
+    k_red_finish<<<1, kFinBlock, 0, ctx->stream>>>(partial, (int)nblk, nr, out, nout, out2, cond, ref, eta, flag);
     CLG_HIP(hipGetLastError());
     return CLG_OK;
 }
@@ -864,7 +845,7 @@ static int multidot_p(clg_context ctx, clg_field_s* const* V, int nv, const clg_
         k_multidot_ch<P><<<dim3(g, nch), kRedBlock, 0, ctx->stream>>>(n, Pn, nv, (const typename Pk<P>::T*)w->data,
                                                                       partial, cond);
         CLG_HIP(hipGetLastError());
-        k_red_finish_ch<<<dim3(1, nch), kRedBlock, 0, ctx->stream>>>(partial, (int)g, nv, out, wnorm, cond);
+        k_red_finish_ch<<<dim3(1, nch), kFinBlock, 0, ctx->stream>>>(partial, (int)g, nv, out, wnorm, cond);
         CLG_HIP(hipGetLastError());
         return CLG_OK;
     }
@@ -1003,19 +984,37 @@ static int gs_step_p(clg_context ctx, clg_field_s* const* V, int nv, clg_field_s
     SWITCH_K(nv, CALL)
 #undef CALL
     CLG_HIP(hipGetLastError());
-    CLG_TRY(red_finish(ctx, g, 2 * nv + 1, hcol, 2 * nv, sc, nullptr, nullptr, 0.0, nullptr));
-    // (2) w' = w - V h with V^H w' and |w'|^2, then the column (or, in the fast form, vnext directly)
     typename Pk<P>::T* vp = vnext ? (typename Pk<P>::T*)vnext->data : nullptr;
-#define CALL(KK)                                                                                     \
-    k_gs_project<P, KK><<<g, kRedBlock, 0, ctx->stream>>>(n, Pp, hcol, wp, ctx->red_partial, sc, vp);  \
-    k_gs_finish<KK><<<1, kRedBlock, 0, ctx->stream>>>(ctx->red_partial, (int)g, hcol, j, shifted ? 1 : 0, sc, vp ? 1 : 0);
+    const int sh = shifted ? 1 : 0;
+    // up to kMergeGrid partial rows every workgroup of the next pass can total them itself, in less time than a
+    // one-workgroup launch takes (3.8 us and a gap); beyond, they come to more L2 reads than that
+    const bool merged = g <= kMergeGrid;
+    double* const p1 = ctx->red_partial;
+    double* const p2 = merged ? p1 + (size_t)kMergeGrid * (2 * kMaxK + 1) : p1;  // read and written by one launch
+    if (!merged) CLG_TRY(red_finish(ctx, g, 2 * nv + 1, hcol, 2 * nv, sc, nullptr, nullptr, 0.0, nullptr));
+    // (2) w' = w - V h with V^H w' and |w'|^2 (or, in the fast form, vnext directly)
+#define CALL(KK)                                                                                                      \
+    if (merged)                                                                                                       \
+        k_gs_project<P, KK, true><<<g, kRedBlock, 0, ctx->stream>>>(n, Pp, hcol, wp, p2, sc, vp, p1, (int)g, j, sh);   \
+    else                                                                                                              \
+        k_gs_project<P, KK, false><<<g, kRedBlock, 0, ctx->stream>>>(n, Pp, hcol, wp, p2, sc, vp, nullptr, 0, j, sh);
     SWITCH_K(nv, CALL)
 #undef CALL
     CLG_HIP(hipGetLastError());
-    // (3) the next basis vector
+    // (3) the column, and the next basis vector
+    if (!merged || !vnext) {
+#define CALL(KK) k_gs_finish<KK><<<1, kFinBlock, 0, ctx->stream>>>(p2, (int)g, hcol, j, sh, sc, vp ? 1 : 0);
+        SWITCH_K(nv, CALL)
+#undef CALL
+        CLG_HIP(hipGetLastError());
+    }
     if (vnext) {
-        const unsigned ge = ew_grid(ctx, n);
-#define CALL(KK) k_gs_finalize<P, KK><<<ge, kRedBlock, 0, ctx->stream>>>(n, Pp, wc, vp, sc);
+#define CALL(KK)                                                                                                      \
+    if (merged)                                                                                                       \
+        k_gs_finalize<P, KK, true><<<g, kRedBlock, 0, ctx->stream>>>(n, Pp, wc, vp, sc, p2, (int)g, hcol, j, sh);      \
+    else                                                                                                              \
+        k_gs_finalize<P, KK, false><<<ew_grid(ctx, n), kRedBlock, 0, ctx->stream>>>(n, Pp, wc, vp, sc, nullptr, 0,     \
+                                                                                    hcol, j, sh);
         SWITCH_K(nv, CALL)
 #undef CALL
         CLG_HIP(hipGetLastError());
@@ -1030,7 +1029,7 @@ int red_finish_partials(clg_context ctx, unsigned nblk, int nr, double* out, int
 }
 int gs_finish_launch(clg_context ctx, unsigned nblk, int nv, double* hcol, int j, bool shifted, double* sc,
                      bool fast_ok) {
-#define CALL(KK) k_gs_finish<KK><<<1, kRedBlock, 0, ctx->stream>>>(ctx->red_partial, (int)nblk, hcol, j, shifted ? 1 : 0, sc, fast_ok ? 1 : 0);
+#define CALL(KK) k_gs_finish<KK><<<1, kFinBlock, 0, ctx->stream>>>(ctx->red_partial, (int)nblk, hcol, j, shifted ? 1 : 0, sc, fast_ok ? 1 : 0);
     SWITCH_K(nv, CALL)
 #undef CALL
     CLG_HIP(hipGetLastError());

@@ -1013,6 +1013,32 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
+// Totals of N per-lane FP64 values over the 64 lanes, written to dst[0..N) (LDS, this wave's row).  N butterflies
+// would take 6 N shuffles; folding halves the values a lane carries at every step (lanes on either side of the
+// exchange keep half of them each), about N + 5 shuffles, after which each lane holds one total.
+template <int N, int OFF>
+__device__ __forceinline__ void wave_fold_step(double* v, int lane, int first, int count, double* dst) {
+    if constexpr (OFF == 0) {
+        if (count > 0) dst[first] = v[0];
+    } else if constexpr (N == 1) {
+        v[0] += __shfl_xor(v[0], OFF, 64);
+        wave_fold_step<1, OFF / 2>(v, lane, first, count, dst);
+    } else {
+        constexpr int H = (N + 1) / 2;
+        const bool up = (lane & OFF) != 0;
+#pragma unroll
+        for (int i = 0; i < H; ++i) {
+            const double lo = v[i], hi = i + H < N ? v[i + H] : 0.0;
+            v[i] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, OFF, 64);
+        }
+        wave_fold_step<H, OFF / 2>(v, lane, up ? first + H : first, up ? max(count - H, 0) : min(count, H), dst);
+    }
+}
+template <int N>
+__device__ __forceinline__ void wave_fold(double (&v)[N], double* dst) {
+    wave_fold_step<N, 32>(v, (int)(threadIdx.x & 63), 0, N, dst);
+}
+
 // Block-level stage of a two-kernel grid reduction: sums NR per-lane FP64 values over the
 // workgroup (blockDim.x <= kRedBlock, a multiple of 64) and writes them to
 // partial[blockIdx.x * NR + r].  No fence or counter: the finishing kernel launched after it on the
@@ -1021,19 +1047,88 @@ __device__ __forceinline__ double wave_sum(double v) {
 template <int NR>
 __device__ void block_partial(double (&v)[NR], double* partial) {
     __shared__ double sm[kRedBlock / 64][NR];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int nw = blockDim.x >> 6;
-#pragma unroll
-    for (int r = 0; r < NR; ++r) v[r] = wave_sum(v[r]);
-    if (lane == 0) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) sm[wv][r] = v[r];
-    }
+    wave_fold<NR>(v, sm[threadIdx.x >> 6]);
     __syncthreads();
     for (int r = threadIdx.x; r < NR; r += blockDim.x) {
         double s = 0;
         for (int w = 0; w < nw; ++w) s += sm[w][r];
         partial[(size_t)blockIdx.x * NR + r] = s;
+    }
+}
+
+// Totals tot[0..nr) (LDS) of nblk x nr row-major partials by one workgroup of BLOCK threads, in a fixed order:
+// thread (q, r) sums value r of blocks q, q + G, ..., neighbouring threads reading neighbouring values, then
+// 8 to 32 strands and one fold the G rows.  nr <= kFinMax.  Measured for 25 values of 24 blocks: the finish 5.5 ->
+// 3.8 us (a thread per block with nr strided accumulators and nr wave butterflies before).
+constexpr int kFinBlock = 1024, kFinMax = 33;
+template <int BLOCK>
+__device__ __forceinline__ void partial_totals(const double* __restrict__ partial, int nblk, int nr, double* tot) {
+    __shared__ double rows[BLOCK];
+    __shared__ double strands[8 * kFinMax];
+    const int G = BLOCK / nr, S = min(G, nr <= 2 ? 32 : nr <= 8 ? 16 : 8), r = (int)threadIdx.x % nr, q = (int)threadIdx.x / nr;
+    double a = 0.0;
+    if (q < G) {
+#pragma unroll 8
+        for (int b = q; b < nblk; b += G) a += partial[(size_t)b * nr + r];
+        rows[threadIdx.x] = a;
+    }
+    __syncthreads();
+    if (q < S) {
+        double t = 0.0;
+        for (int i = q; i < G; i += S) t += rows[i * nr + r];
+        strands[threadIdx.x] = t;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < nr) {
+        double t = 0.0;
+        for (int i = 0; i < S; ++i) t += strands[i * nr + threadIdx.x];
+        tot[threadIdx.x] = t;
+    }
+    __syncthreads();
+}
+
+// Least-squares solution of the (m+1) x m Hessenberg system H y = sqrt(beta2) e_1 by one wave (m <= 64): Givens
+// rotations and back substitution as RotateH / SolveY (CSolverGMRES.cpp:262-358), FP64.  H is column-major with
+// leading dimension ld; sm holds m * ld complex numbers of LDS.  Lane j carries column j: a rotation is one
+// broadcast and four products a lane, and the back substitution eliminates column by column.  dev[0] = |g_m|^2,
+// dev[1] = |g_m|.  Measured for m = 12: 7.7 us (one thread on
+// global memory: 28).
+__device__ __forceinline__ cd lane_bcast(cd a, int src) { return cd{__shfl(a.x, src, 64), __shfl(a.y, src, 64)}; }
+__device__ __forceinline__ void gmres_lsq_wave(const double* __restrict__ H, int ld, int m, double beta2, double* y,
+                                               double* dev, cd* sm) {
+    const int lane = (int)(threadIdx.x & 63), col = min(lane, m - 1);
+    for (int i = lane; i < m * ld; i += 64) sm[i] = cd{H[2 * i], H[2 * i + 1]};
+    __syncthreads();
+    cd cur = sm[col * ld], g = cd{sqrt(beta2), 0.0}, z = cd{0.0, 0.0};
+    for (int k = 0; k < m; ++k) {
+        const cd nxt = sm[col * ld + k + 1];  // below the subdiagonal of columns < k: not used
+        const cd hkk = lane_bcast(cur, k), hk1 = lane_bcast(nxt, k);
+        const double den = 1.0 / sqrt(hkk.x * hkk.x + hkk.y * hkk.y + hk1.x * hk1.x + hk1.y * hk1.y);
+        const cd cs = cscale(hkk, den), sn = cscale(hk1, den);
+        const cd gk = cmul(cconj(cs), g);
+        g = cmul(sn, cd{-g.x, -g.y});
+        if (lane == k) z = gk;
+        if (lane >= k && lane < m) {
+            sm[col * ld + k] = cadd(cmul(cconj(cs), cur), cmul(cconj(sn), nxt));
+            cur = csub(cmul(cs, nxt), cmul(sn, cur));
+        }
+    }
+    if (lane == 0) {
+        dev[0] = g.x * g.x + g.y * g.y;
+        dev[1] = sqrt(dev[0]);
+    }
+    __syncthreads();
+    for (int k = m - 1; k >= 0; --k) {
+        const cd d = sm[k * ld + k], acc = lane_bcast(z, k);
+        const double dd = d.x * d.x + d.y * d.y;
+        const cd yk = cd{(acc.x * d.x + acc.y * d.y) / dd, (acc.y * d.x - acc.x * d.y) / dd};
+        if (lane == k) z = yk;
+        else if (lane < k) z = csub(z, cmul(sm[k * ld + lane], yk));
+    }
+    if (lane < m) {
+        y[2 * lane] = z.x;
+        y[2 * lane + 1] = z.y;
     }
 }
 

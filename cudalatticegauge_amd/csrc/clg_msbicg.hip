@@ -104,13 +104,7 @@ __device__ __forceinline__ void cdot(double* acc, const double* a, const double*
 template <int NR>
 __device__ void bcg_partial(double (&v)[NR], double* part) {
     __shared__ double sm[kBcgBlock / 64][NR];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-    for (int r = 0; r < NR; ++r) v[r] = wave_sum(v[r]);
-    if (lane == 0) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) sm[wv][r] = v[r];
-    }
+    wave_fold<NR>(v, sm[threadIdx.x >> 6]);
     __syncthreads();
     for (int r = threadIdx.x; r < NR; r += blockDim.x) {
         double s = 0.0;

@@ -49,40 +49,10 @@ int gauge_convert(clg_context, clg_field_s* dst, const clg_field_s* src);
 namespace {
 
 // ------------------------------------------------------------------ small device kernels
-// Givens rotations of the (m+1) x m Hessenberg matrix with g = beta e1 and back
-// substitution (RotateH / SolveY, CSolverGMRES.cpp:262-358), FP64, one thread.
-// out: y[0..m), dev[0] = |g_m|^2, dev[1] = |g_m|
-__global__ void k_gmres_lsq(double* H, int ld, int m, const double* beta2, double* g, double* y, double* dev) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    typedef C2<double> c;
-    auto Hp = [&](int r, int col) -> c* { return reinterpret_cast<c*>(H + 2 * (col * ld + r)); };
-    c* G = reinterpret_cast<c*>(g);
-    c* Y = reinterpret_cast<c*>(y);
-    G[0] = c{sqrt(beta2[0]), 0.0};
-    for (int k = 1; k <= m; ++k) G[k] = c{0.0, 0.0};
-    for (int k = 0; k < m; ++k) {
-        const c hkk = *Hp(k, k), hk1 = *Hp(k + 1, k);
-        const double den = 1.0 / sqrt(hkk.x * hkk.x + hkk.y * hkk.y + hk1.x * hk1.x + hk1.y * hk1.y);
-        const c cs = cscale(hkk, den), sn = cscale(hk1, den);
-        const c csh = cconj(cs), snh = cconj(sn);
-        for (int j = k; j < m; ++j) {
-            const c hkj = *Hp(k, j), h1j = *Hp(k + 1, j);
-            *Hp(k, j) = cadd(cmul(csh, hkj), cmul(snh, h1j));
-            *Hp(k + 1, j) = csub(cmul(cs, h1j), cmul(sn, hkj));
-        }
-        const c mg = c{-G[k].x, -G[k].y};
-        G[k] = cmul(csh, G[k]);
-        G[k + 1] = cmul(sn, mg);
-    }
-    dev[0] = G[m].x * G[m].x + G[m].y * G[m].y;
-    dev[1] = sqrt(dev[0]);
-    for (int k = m - 1; k >= 0; --k) {
-        c acc = G[k];
-        for (int j = k + 1; j < m; ++j) acc = csub(acc, cmul(*Hp(k, j), Y[j]));
-        const c d = *Hp(k, k);
-        const double dd = d.x * d.x + d.y * d.y;
-        Y[k] = c{(acc.x * d.x + acc.y * d.y) / dd, (acc.y * d.x - acc.x * d.y) / dd};
-    }
+// y of the cycle's least-squares problem and its residual: dev[0] = |g_m|^2, dev[1] = |g_m|
+__global__ __launch_bounds__(64) void k_gmres_lsq(const double* H, int ld, int m, const double* beta2, double* y, double* dev) {
+    extern __shared__ cd sm[];
+    gmres_lsq_wave(H, ld, m, beta2[0], y, dev, sm);
 }
 
 // BiCGStab scalar updates (all FP64 on device).  s[] layout:
@@ -217,13 +187,11 @@ int gmres(clg_context ctx, LinOp& A, clg_field_s* x, const clg_field_s* b, int m
         CLG_TRY(scratch_field(ctx, b, b->kind, b->prec, b->subset, 1000 + k, &V[k]));
     clg_field_s* w = V[m];
     const int ld = m + 1;
-    // device workspace: H, c2, g, y, scalars
-    const size_t offH = 0, offC = offH + 2 * (size_t)ld * m, offG = offC + 2 * (size_t)m,
-                 offY = offG + 2 * (size_t)(m + 1), offS = offY + 2 * (size_t)m, offGS = offS + 16;
+    // device workspace: H, y, scalars
+    const size_t offH = 0, offY = offH + 2 * (size_t)ld * m, offS = offY + 2 * (size_t)m, offGS = offS + 16;
     double* wsp = nullptr;
     CLG_TRY(workspace(ctx, offGS + kArnScratch, &wsp));
     double* H = wsp + offH;
-    double* g = wsp + offG;
     double* y = wsp + offY;
     double* sc = wsp + offS;  // sc[0] |r|^2, sc[1] |w|^2, sc[2..3] deviation, sc[4] |w|^2 before GS
     const bool shifted = A.shiftable();
@@ -259,7 +227,10 @@ int gmres(clg_context ctx, LinOp& A, clg_field_s* x, const clg_field_s* b, int m
             }
             CLG_TRY(arn_step(ctx, V.data(), j + 1, w, Hj, j, shifted, j < m - 1 ? V[j + 1] : nullptr, wsp + offGS));
         }
-        k_gmres_lsq<<<1, 64, 0, ctx->stream>>>(H, ld, m, sc, g, y, sc + 2);
+        const size_t lsq_bytes = sizeof(cd) * (size_t)m * ld;  // over 64 KiB only for m = 64
+        if (lsq_bytes > 65536)
+            CLG_HIP(hipFuncSetAttribute((const void*)k_gmres_lsq, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lsq_bytes));
+        k_gmres_lsq<<<1, 64, lsq_bytes, ctx->stream>>>(H, ld, m, sc, y, sc + 2);
         CLG_HIP(hipGetLastError());
         CLG_TRY(blas_multiaxpy_dev(ctx, x, V.data(), m, y, 1.0, nullptr, nullptr, nullptr, 0.0, nullptr));
         x_is_zero = false;

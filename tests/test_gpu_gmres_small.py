@@ -1,0 +1,57 @@
+"""GMRES on both sides of the size up to which the Gram-Schmidt passes total the projections themselves, through
+the fast form (Wilson D, whose steps run on 1 - D) and the general one with its second pass (D D^dagger,
+staggered D), and Krylov dimensions at the edges of the least-squares kernel."""
+import numpy as np
+import pytest
+
+import cudalatticegauge_amd as clg
+import orc
+
+pytestmark = pytest.mark.gpu
+
+# 4 x 12 complex numbers a site of parity: 49152, 65520 (the last merged size is 65536) and 73728 of them
+LATTICES = [(8, 8, 8, 8), (5, 6, 13, 14), (8, 8, 8, 12)]
+
+
+def put(ctx, kind, prec, dims, data):
+    f = clg.Field(ctx, kind, prec, dims, bc=None if kind == clg.GAUGE else orc.BC_FERMION)
+    f.upload(data)
+    return f
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = clg.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("dims", LATTICES)
+@pytest.mark.parametrize("prec,acc", [(clg.F64, 1e-11), (clg.F32, 2e-6)])
+def test_solves(ctx, dims, prec, acc):
+    U = orc.gauge_random(dims, 0.3, 1)
+    g = put(ctx, clg.GAUGE, prec, dims, U)
+    for kind, m, op, oop, b in ((clg.WILSON, 0.13, clg.EFO_F_D, orc.D, orc.wilson_gaussian(dims, 2)),
+                                (clg.WILSON, 0.05, clg.EFO_F_DDdagger, orc.DDDAG, orc.wilson_gaussian(dims, 3)),
+                                (clg.KS, 1.5, clg.EFO_F_D, orc.D, orc.ks_gaussian(dims, 4))):
+        x = clg.Field(ctx, kind, prec, dims, bc=orc.BC_FERMION)
+        for max_dim in (1, 12, 16):
+            p = clg.solver_params(kind=kind, max_dim=max_dim, restart=2000, accuracy=acc,
+                                  stop_rule=clg.STOP_TRUE_RESIDUAL, even_odd=0)
+            st, rep = clg.solve(ctx, p, x, put(ctx, kind, prec, dims, b), g, m, op)
+            apply = orc.wilson_op if kind == clg.WILSON else orc.ks_op
+            r = apply(dims, orc.BC_FERMION, m, U, x.download(), oop) - b
+            res = np.linalg.norm(r) / np.linalg.norm(b)
+            # the solver's own residual, plus the rounding of x and U to FP32 (2^-24 times |D||x|/|b| < 8)
+            assert st == clg.OK and res < acc * 1.01 + (1e-6 if prec == clg.F32 else 1e-14), (kind, op, max_dim, res)
+
+
+@pytest.mark.parametrize("max_dim", [17, 64])
+def test_long_bases(ctx, max_dim):
+    dims = (4, 4, 4, 6)
+    U, b = orc.gauge_random(dims, 0.3, 1), orc.wilson_gaussian(dims, 2)
+    g, x = put(ctx, clg.GAUGE, clg.F64, dims, U), clg.Field(ctx, clg.WILSON, clg.F64, dims, bc=orc.BC_FERMION)
+    p = clg.solver_params(max_dim=max_dim, restart=20, accuracy=1e-11, stop_rule=clg.STOP_TRUE_RESIDUAL, even_odd=0)
+    st, _ = clg.solve(ctx, p, x, put(ctx, clg.WILSON, clg.F64, dims, b), g, 0.13, clg.EFO_F_D)
+    r = orc.wilson_op(dims, orc.BC_FERMION, 0.13, U, x.download()) - b
+    assert st == clg.OK and np.linalg.norm(r) < 1.01e-11 * np.linalg.norm(b)
