@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <functional>
@@ -207,6 +208,56 @@ void tune_cache_append(const std::string& path, const char* tuner, const std::ve
 int ks_tune_count();
 int ks_tune_entry(int index, char* buf, int len);
 void ks_tune_reset();
+
+// Times the candidate launches of one operator call on its stream (every candidate writes the same output) and
+// returns the fastest in `best`, its time in `best_ms` (milliseconds a launch).  A first round of a warm-up and
+// three launches each; then those within 15 % of the fastest, six at most, are timed in turn three times over 20
+// launches or about 1 ms, and the sum counts: three launches are within the noise of the clocks and of what ran
+// before them.
+template <class C, class L, class V>
+int tune_pick(hipStream_t st, const std::vector<C>& cands, L launch, V report, C& best, float& best_ms) {
+    hipEvent_t e0, e1;
+    CLG_HIP(hipEventCreate(&e0));
+    CLG_HIP(hipEventCreate(&e1));
+    auto timed = [&](const C& c, int reps, float& ms) -> int {
+        CLG_HIP(hipEventRecord(e0, st));
+        for (int r = 0; r < reps; ++r) CLG_TRY(launch(c));
+        CLG_HIP(hipEventRecord(e1, st));
+        CLG_HIP(hipEventSynchronize(e1));
+        CLG_HIP(hipEventElapsedTime(&ms, e0, e1));
+        ms /= (float)reps;
+        return CLG_OK;
+    };
+    std::vector<std::pair<float, size_t>> t;
+    int status = CLG_OK;
+    for (size_t i = 0; i < cands.size() && status == CLG_OK; ++i) {
+        float ms = 0.f;
+        status = launch(cands[i]);  // warm
+        if (status == CLG_OK) status = timed(cands[i], 3, ms);
+        t.emplace_back(ms, i);
+        report(cands[i], ms);
+    }
+    std::sort(t.begin(), t.end());
+    size_t near = 0;
+    while (near < t.size() && near < 6 && t[near].first <= 1.15f * t[0].first) ++near;
+    std::vector<float> sum(near, 0.f);
+    for (int round = 0; round < 3 && near > 1; ++round)
+        for (size_t q = 0; q < near && status == CLG_OK; ++q) {
+            float ms = 0.f;
+            const int reps = std::max(3, std::min(20, (int)(1.f / std::max(t[0].first, 1e-4f))));
+            status = timed(cands[t[q].second], reps, ms);
+            sum[q] += ms / 3.f;
+        }
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    CLG_TRY(status);
+    size_t q = 0;
+    for (size_t k = 1; k < near && near > 1; ++k)
+        if (sum[k] < sum[q]) q = k;
+    best = cands[t[q].second];
+    best_ms = near > 1 ? sum[q] : t[q].first;
+    return CLG_OK;
+}
 
 // launch helpers
 inline unsigned grid_for(long n, int block) { return (unsigned)((n + block - 1) / block); }

@@ -365,38 +365,25 @@ int ks_launch(const KSArgs& a, int prec, int gprec, bool r12, hipStream_t st) {
         std::vector<KSCfg> cands = {{64, 0, 2}, {128, 0, 2}, {256, 0, 2}, {64, 8, 2}, {128, 8, 2}, {256, 8, 2},
                                {64, 8, 0}, {128, 8, 0}, {256, 8, 0},
                                {kSplitSites, 0, kSplitPm}, {kSplitSites, 8, kSplitPm}};
-        hipEvent_t e0, e1;
-        CLG_HIP(hipEventCreate(&e0));
-        CLG_HIP(hipEventCreate(&e1));
-        float best = 1e30f;
         for (int TY : {2, 4, 8})
             if (tile64_fits(a.g, TY))
                 for (int m : {0, 1}) cands.push_back(KSCfg{kSplitSites, 10 * TY + m, kSplitPm});
-        for (const KSCfg& c : cands) {
-            CLG_TRY(ks_launch_cfg(a, prec, gprec, r12, st, c));  // warm
-            float ms = 0.f;  // of three launches
-            // a launch of a few microseconds is timed again over more of them: three are within the clock's noise
-            for (int reps : {3, 15}) {
-                if (reps == 15 && (ms > 0.12f || ms > 1.3f * best)) break;
-                CLG_HIP(hipEventRecord(e0, st));
-                for (int r = 0; r < reps; ++r) CLG_TRY(ks_launch_cfg(a, prec, gprec, r12, st, c));
-                CLG_HIP(hipEventRecord(e1, st));
-                CLG_HIP(hipEventSynchronize(e1));
-                CLG_HIP(hipEventElapsedTime(&ms, e0, e1));
-                ms *= 3.f / (float)reps;
-            }
-            if (ms < best) { best = ms; cfg = c; }
-            const char* v2 = std::getenv("CLG_TUNE_VERBOSE");
-            if (v2 && v2[0] == '2')  // every candidate
-                std::fprintf(stderr, "[clg tune]   candidate pin=%d block=%d xcd=%d: %.1f us\n", c.pm, c.block, c.xcd, ms * 1e3 / 3);
-        }
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
+        float best = 0.f;
+        const char* v2 = std::getenv("CLG_TUNE_VERBOSE");
+        const bool each = v2 && v2[0] == '2';
+        CLG_TRY(tune_pick(
+            st, cands, [&](const KSCfg& c) { return ks_launch_cfg(a, prec, gprec, r12, st, c); },
+            [&](const KSCfg& c, float ms) {
+                if (each)
+                    std::fprintf(stderr, "[clg tune]   candidate pin=%d block=%d xcd=%d: %.1f us\n", c.pm, c.block, c.xcd,
+                                 ms * 1e3);
+            },
+            cfg, best));
         const char* verbose = std::getenv("CLG_TUNE_VERBOSE");
         if (verbose && (verbose[0] == '1' || verbose[0] == '2'))
             std::fprintf(stderr, "[clg tune] staggered D prec=%d gprec=%d recon=%d mode=%d L=%dx%dx%dx%d -> block=%d xcd=%d pin=%d (%.1f us)\n",
                          prec, gprec, r12 ? 12 : 18, a.mode, a.g.L[0], a.g.L[1], a.g.L[2], a.g.L[3], cfg.block, cfg.xcd,
-                         cfg.pm, best * 1e3 / 3);
+                         cfg.pm, best * 1e3);
         std::lock_guard<std::mutex> lk(ks_mutex());
         ks_table()[k] = cfg;
         tune_cache_append(cpath, "staggered_d", {k.prec, k.gprec, k.r12, k.mode, k.L0, k.L1, k.L2, k.L3},

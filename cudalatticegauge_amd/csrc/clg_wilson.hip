@@ -535,10 +535,6 @@ int launch_hop(const HopArgs& a, int prec, int gprec, int recon, bool dag, bool 
         const HopCfg cands[] = {{1, 64, 0}, {1, 128, 0}, {1, 256, 0}, {2, 64, 0}, {2, 128, 0}, {2, 256, 0},
                                 {1, 64, 8}, {1, 128, 8}, {1, 256, 8}, {2, 64, 8}, {2, 128, 8}, {2, 256, 8},
                                 {3, 64, 8}, {3, 128, 8}, {3, 256, 8}, {4, 64, 8}, {4, 128, 8}, {4, 256, 8}};
-        hipEvent_t e0, e1;
-        CLG_HIP(hipEventCreate(&e0));
-        CLG_HIP(hipEventCreate(&e1));
-        float best = 1e30f;
         std::vector<HopCfg> all(std::begin(cands), std::end(cands));
         // several sites per thread for the XCD-slab launches
         for (int spt : {2, 4})
@@ -568,32 +564,30 @@ int launch_hop(const HopArgs& a, int prec, int gprec, int recon, bool dag, bool 
                             if (m == 0 && TY >= 4) all.push_back(HopCfg{pm, sb, 10 * TY + m, 1, 1});
                         }
         }
-        for (const HopCfg& c : all) {
-            CLG_TRY(launch_cfg(a, prec, gprec, recon, dag, hasx, st, c));  // warm
-            float ms = 0.f;  // of three launches
-            // a launch of a few microseconds is timed again over more of them: three are within the clock's noise
-            for (int reps : {3, 15}) {
-                if (reps == 15 && (ms > 0.12f || ms > 1.3f * best)) break;
-                CLG_HIP(hipEventRecord(e0, st));
-                for (int r = 0; r < reps; ++r) CLG_TRY(launch_cfg(a, prec, gprec, recon, dag, hasx, st, c));
-                CLG_HIP(hipEventRecord(e1, st));
-                CLG_HIP(hipEventSynchronize(e1));
-                CLG_HIP(hipEventElapsedTime(&ms, e0, e1));
-                ms *= 3.f / (float)reps;
-            }
-            if (ms < best) { best = ms; cfg = c; }
-            const char* v2 = std::getenv("CLG_TUNE_VERBOSE");
-            if (v2 && v2[0] == '2')  // every candidate
-                std::fprintf(stderr, "[clg tune]   candidate pin=%d block=%d xcd=%d spt=%d nt=%d: %.1f us\n", c.pm,
-                             c.block, c.xcd, c.spt, c.nt, ms * 1e3 / 3);
-        }
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
+        // Links that fit the 32 MB of L2 are read from there by the next hops: no non-temporal loads of them.  The
+        // tuner's own launches cannot show it (FP32 half hops at 16^4 in a solve: 6.6 us, non-temporal 9.4).
+        if (8L * a.g.Vh * (recon == 12 ? 12 : 18) * (gprec == CLG_F64 ? 8 : gprec == CLG_F32 ? 4 : 2) <= (32L << 20))
+            all.erase(std::remove_if(all.begin(), all.end(),
+                                     [](const HopCfg& c) {
+                                         return c.pm == 3 || c.pm == 4 || c.pm == 7 || c.pm == 8 || c.pm == kSplitNtPm;
+                                     }),
+                      all.end());
+        float best = 0.f;
+        const char* v2 = std::getenv("CLG_TUNE_VERBOSE");
+        const bool each = v2 && v2[0] == '2';
+        CLG_TRY(tune_pick(
+            st, all, [&](const HopCfg& c) { return launch_cfg(a, prec, gprec, recon, dag, hasx, st, c); },
+            [&](const HopCfg& c, float ms) {
+                if (each)
+                    std::fprintf(stderr, "[clg tune]   candidate pin=%d block=%d xcd=%d spt=%d nt=%d: %.1f us\n", c.pm,
+                                 c.block, c.xcd, c.spt, c.nt, ms * 1e3);
+            },
+            cfg, best));
         const char* verbose = std::getenv("CLG_TUNE_VERBOSE");
         if (verbose && (verbose[0] == '1' || verbose[0] == '2'))
             std::fprintf(stderr, "[clg tune] wilson hop prec=%d gprec=%d recon=%d dag=%d x=%d nblk=%d L=%dx%dx%dx%d -> pin=%d block=%d xcd=%d spt=%d nt=%d (%.1f us)\n",
                          prec, gprec, recon, (int)dag, (int)hasx, a.nblk, a.g.L[0], a.g.L[1], a.g.L[2], a.g.L[3],
-                         cfg.pm, cfg.block, cfg.xcd, cfg.spt, cfg.nt, best * 1e3 / 3);
+                         cfg.pm, cfg.block, cfg.xcd, cfg.spt, cfg.nt, best * 1e3);
         std::lock_guard<std::mutex> lk(tune_mutex());
         tune_table()[k] = cfg;
         tune_cache_append(cpath, "wilson_hop", key_vec(k), {cfg.pm, cfg.block, cfg.xcd, cfg.spt, cfg.nt});
