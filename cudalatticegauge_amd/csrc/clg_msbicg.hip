@@ -4,18 +4,24 @@
 // The reference keeps delta, phi, beta, alpha, chi and the per-shift zeta / beta / alpha / chi / rho
 // recurrences on the host and reads four inner products back per step.  Here a step is a fixed
 // sequence of launches with no host wait (state: kBcgState doubles of the context workspace):
+//   [phi = <W0, SA> / delta, beta; per shift zeta, beta_k (:218, :133-164)]
 //   W  = R + beta SA                                     k_bcg_w             (:166-167)
 //   WA = A W                                             operator            (:168-169)
 //   partials of <WA, W> and |WA|^2                       k_bcg_dot<P, true>
-//   chi; per shift chi_k, the first update's coefficients, rho_k        fin (:170-190)
+//   [chi; per shift chi_k, the first update's coefficients, rho_k (:170-190)]
 //   per active shift x_k += -beta_k s_k + (chi rho zeta)_k W,
 //     s_k += -(chi rho zeta / beta)_k W + (chi rho zeta_old / beta)_k R;
 //   R = W - chi WA; partials of <W0, R>                  k_bcg_upd1          (:182-194)
-//   delta', alpha, delta; per shift alpha_k, the second update's coefficients   fin (:195-206)
+//   [delta', alpha, delta; per shift alpha_k, the second update's coefficients (:195-206)]
 //   S = alpha (S - chi SA) + R                           k_bcg_upd2          (:212-214)
 //   SA = A S                                             operator            (:216-217)
 //   partials of <W0, SA>                                 k_bcg_dot<P, false>
-//   phi = <W0, SA> / delta; the next step's beta and per-shift zeta, beta_k      fin (:218, :133-164)
+// The scalar stages in brackets run at the start of the kernel named below them: every workgroup totals the
+// partials and computes the scalars it needs, workgroup 0 stores the state.  A stage therefore stores nothing that
+// another workgroup of its own launch reads: what a later launch needs of a scalar that is still read goes to a
+// second slot (delta, rho_k).  The last step's phi stage runs with the next group's first step.  Measured, us a
+// step: 24^3x8 with 12 shifts in FP32 76.5 -> 73.8, 12x12x10x14 with 7 in FP64 46 -> 41, against three
+// one-workgroup launches a step.
 // so DiviationStep steps replay as one recorded graph.  The check after them (|S| and |s_k| of the
 // shifts still active, :220-242) is one more reduction and the only read back to the host; a shift
 // whose |s_k| fell below the bound leaves the active set on the device.  The per-shift vector updates
@@ -56,17 +62,17 @@ constexpr int kBcgNormRows = kBcgMaxShift + 1;
 
 // device state (doubles): globals, then per-shift arrays of kBcgMaxShift entries
 enum : int {
-    kDelta = 0, kPhi = 2, kBeta = 4, kAlpha = 6, kChi = 8, kMaxErr = 10, kDone = 11,
+    kDelta = 0, kPhi = 2, kBeta = 4, kAlpha = 6, kChi = 8, kMaxErr = 10, kDone = 11, kDeltaNext = 12,
     oCn = 16,
     oZeta = oCn + 2 * kBcgMaxShift,
     oZold = oZeta + 2 * kBcgMaxShift,
     oBetas = oZold + 2 * kBcgMaxShift,
     oRho = oBetas + 2 * kBcgMaxShift,
-    oC8 = oRho + 2 * kBcgMaxShift,
-    oC4 = oC8 + 8 * kBcgMaxShift,
+    oC4 = oRho + 2 * kBcgMaxShift,
     oSl = oC4 + 4 * kBcgMaxShift,
     oAct = oSl + kBcgMaxShift,
-    kBcgState = oAct + kBcgMaxShift
+    oRhoNext = oAct + kBcgMaxShift,
+    kBcgState = oRhoNext + 2 * kBcgMaxShift
 };
 
 struct dcx {
@@ -118,19 +124,113 @@ struct BcgShifts {
     void* s[kBcgMaxShift];
 };
 
+// ---- the scalar stages, by every thread of a workgroup (thread k < ns: shift k) from the totals tot; `store`: this
+// workgroup keeps the state
+// phi = <W0, SA> / delta (:218); the step's newbeta = -1 / phi and per-shift zeta, beta_k (:133-164), then beta =
+// newbeta, which is returned
+__device__ __forceinline__ dcx stage_phi(const double* tot, double* st, int ns, int first, bool store) {
+    const dcx delta = ld2(st + kDeltaNext);
+    const dcx phi = cdiv(dcx{tot[0], tot[1]}, delta);
+    const dcx nb = cdiv(dcx{-1.0, 0.0}, phi);
+    if (store) {
+        const int t = threadIdx.x;
+        if (t < ns && st[oAct + t] != 0.0) {
+            const dcx cn = ld2(st + oCn + 2 * t);
+            const dcx one_cnb = csub(dcx{1.0, 0.0}, cmul(cn, nb));
+            if (first) {
+                const dcx z = cdiv(dcx{1.0, 0.0}, one_cnb);
+                st2(st + oZeta + 2 * t, z);
+                st2(st + oBetas + 2 * t, cmul(nb, z));
+            } else {
+                const dcx beta = ld2(st + kBeta), alpha = ld2(st + kAlpha);
+                const dcx znm1 = ld2(st + oZold + 2 * t);
+                const dcx zold = ld2(st + oZeta + 2 * t);
+                const dcx zb = cmul(znm1, beta);
+                const dcx z = cdiv(cmul(zold, zb), cadd(cmul(alpha, cmul(nb, csub(znm1, zold))), cmul(zb, one_cnb)));
+                st2(st + oZold + 2 * t, zold);
+                st2(st + oZeta + 2 * t, z);
+                st2(st + oBetas + 2 * t, cdiv(cmul(nb, z), zold));
+            }
+        }
+        __syncthreads();  // every shift has read beta
+        if (t == 0) {
+            st2(st + kPhi, phi);
+            st2(st + kBeta, nb);
+            st2(st + kDelta, delta);
+        }
+    }
+    return nb;
+}
+// chi = <WA, W> / |WA|^2 (:170), returned, and per shift the first update's coefficients to c8 (LDS) and rho (:178-189)
+__device__ __forceinline__ dcx stage_chi(const double* tot, double* st, int ns, double* c8, bool store) {
+    const dcx chi = {tot[0] / tot[2], tot[1] / tot[2]};
+    const int t = threadIdx.x;
+    if (t < ns && st[oAct + t] != 0.0) {
+        const dcx cn = ld2(st + oCn + 2 * t);
+        const dcx dinom = cadd(dcx{1.0, 0.0}, cmul(cn, chi));
+        const dcx chis = cdiv(chi, dinom);
+        const dcx rho = ld2(st + oRho + 2 * t);
+        const dcx betas = ld2(st + oBetas + 2 * t);
+        const dcx chirho = cmul(chis, rho);
+        const dcx crz = cmul(chirho, ld2(st + oZeta + 2 * t));
+        const dcx crzb = cdiv(crz, betas);
+        const dcx crzob = cdiv(cmul(chirho, ld2(st + oZold + 2 * t)), betas);
+        double* c = c8 + 8 * t;
+        c[0] = -betas.x;
+        c[1] = -betas.y;
+        c[2] = crz.x;
+        c[3] = crz.y;
+        c[4] = -crzb.x;
+        c[5] = -crzb.y;
+        c[6] = crzob.x;
+        c[7] = crzob.y;
+        if (store) st2(st + oRhoNext + 2 * t, cdiv(rho, dinom));
+    }
+    if (store && t == 0) st2(st + kChi, chi);
+    return chi;
+}
+// delta' = <W0, R>, alpha = beta (-delta') / (chi delta), returned, delta = delta' (:194-196); per shift alpha_k and the
+// second update's coefficients (:205-209)
+__device__ __forceinline__ dcx stage_alpha(const double* tot, double* st, int ns, bool store) {
+    const dcx nd = {tot[0], tot[1]};
+    const dcx beta = ld2(st + kBeta);
+    const dcx alpha = cdiv(cmul(beta, dcx{-nd.x, -nd.y}), cmul(ld2(st + kChi), ld2(st + kDelta)));
+    if (store) {
+        const int t = threadIdx.x;
+        if (t < ns && st[oAct + t] != 0.0) {
+            const dcx z = ld2(st + oZeta + 2 * t), rho = ld2(st + oRhoNext + 2 * t);
+            const dcx as = cdiv(cmul(cmul(alpha, z), ld2(st + oBetas + 2 * t)), cmul(ld2(st + oZold + 2 * t), beta));
+            const dcx zr = cmul(z, rho);
+            double* c = st + oC4 + 4 * t;
+            c[0] = as.x;
+            c[1] = as.y;
+            c[2] = zr.x;
+            c[3] = zr.y;
+            st2(st + oRho + 2 * t, rho);
+        }
+        if (t == 0) {
+            st2(st + kAlpha, alpha);
+            st2(st + kDeltaNext, nd);
+        }
+    }
+    return alpha;
+}
+
 // W = R + beta SA
 template <int P>
-__global__ __launch_bounds__(kBcgBlock) void k_bcg_w(long n, const double* __restrict__ st,
-                                                     const typename Pk<P>::T* __restrict__ R,
+__global__ __launch_bounds__(kBcgBlock) void k_bcg_w(long n, int ns, double* st, const double* __restrict__ part, int G,
+                                                     int first, const typename Pk<P>::T* __restrict__ R,
                                                      const typename Pk<P>::T* __restrict__ SA,
                                                      typename Pk<P>::T* __restrict__ W) {
     constexpr int NC = Pk<P>::NC;
-    const dcx beta = ld2(st + kBeta);
+    __shared__ double tot[kFinMax];
+    partial_totals<kBcgBlock>(part, G, 2, tot);
+    const dcx nb = stage_phi(tot, st, ns, first, blockIdx.x == 0);
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
         double r[2 * NC], sa[2 * NC];
         Pk<P>::ld(R, i, r);
         Pk<P>::ld(SA, i, sa);
-        cmad<NC>(r, beta, sa);
+        cmad<NC>(r, nb, sa);
         Pk<P>::st(W, i, r);
     }
 }
@@ -160,8 +260,11 @@ __global__ __launch_bounds__(kBcgBlock) void k_bcg_dot(long n, const typename Pk
 // the first update of every active shift, R = W - chi WA, partials of <W0, R>.  s_k is stored as it was
 // before the previous step's second update s_k <- alpha_k s_k + (zeta rho)_k R (coefficients c4, R the
 // vector this kernel reads before it overwrites it), which is applied here on the fly.
+// Bound by the x_k and s_k, 127 MB read and written at 24^3x8 with 12 shifts in FP32: 19 us, 6.7 TB/s (with
+// non-temporal accesses the solve takes 4 % longer).
 template <int P>
-__global__ __launch_bounds__(kBcgBlock) void k_bcg_upd1(long n, int ns, BcgShifts sp, const double* __restrict__ st,
+__global__ __launch_bounds__(kBcgBlock) void k_bcg_upd1(long n, int ns, BcgShifts sp, double* st,
+                                                        const double* __restrict__ pin, int G,
                                                         const typename Pk<P>::T* __restrict__ W,
                                                         const typename Pk<P>::T* __restrict__ WA,
                                                         const typename Pk<P>::T* __restrict__ W0,
@@ -171,11 +274,13 @@ __global__ __launch_bounds__(kBcgBlock) void k_bcg_upd1(long n, int ns, BcgShift
     __shared__ double cs[8 * kBcgMaxShift];
     __shared__ double c2[4 * kBcgMaxShift];
     __shared__ int act[kBcgMaxShift];
-    for (int t = threadIdx.x; t < 8 * ns; t += blockDim.x) cs[t] = st[oC8 + t];
     for (int t = threadIdx.x; t < 4 * ns; t += blockDim.x) c2[t] = st[oC4 + t];
     for (int t = threadIdx.x; t < ns; t += blockDim.x) act[t] = st[oAct + t] != 0.0;
+    __shared__ double tot[kFinMax];
+    partial_totals<kBcgBlock>(pin, G, 3, tot);
+    const dcx chi = stage_chi(tot, st, ns, cs, blockIdx.x == 0);
     __syncthreads();
-    const dcx mchi = {-st[kChi], -st[kChi + 1]};
+    const dcx mchi = {-chi.x, -chi.y};
     double v[2] = {0.0, 0.0};
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
         double w[2 * NC], r[2 * NC];
@@ -227,13 +332,16 @@ __global__ __launch_bounds__(kBcgBlock) void k_bcg_upd1(long n, int ns, BcgShift
 
 // S = alpha (S - chi SA) + R
 template <int P>
-__global__ __launch_bounds__(kBcgBlock) void k_bcg_upd2(long n, const double* __restrict__ st,
+__global__ __launch_bounds__(kBcgBlock) void k_bcg_upd2(long n, int ns, double* st, const double* __restrict__ part, int G,
                                                         const typename Pk<P>::T* __restrict__ R,
                                                         const typename Pk<P>::T* __restrict__ SA,
                                                         typename Pk<P>::T* __restrict__ S) {
     constexpr int NC = Pk<P>::NC;
-    const dcx mchi = {-st[kChi], -st[kChi + 1]};
-    const dcx alpha = ld2(st + kAlpha);
+    const dcx chi = ld2(st + kChi);
+    __shared__ double tot[kFinMax];
+    partial_totals<kBcgBlock>(part, G, 2, tot);
+    const dcx alpha = stage_alpha(tot, st, ns, blockIdx.x == 0);
+    const dcx mchi = {-chi.x, -chi.y};
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
         double r[2 * NC], s[2 * NC], sa[2 * NC];
         Pk<P>::ld(R, i, r);
@@ -284,43 +392,21 @@ __global__ __launch_bounds__(kBcgBlock) void k_bcg_norms(long n, int ns, BcgShif
     bcg_partial<kBcgNormRows>(v, part);
 }
 
-enum { FIN_INIT = 0, FIN_PHI = 1, FIN_CHI = 2, FIN_ALPHA = 3, FIN_CHECK = 4 };
+enum { FIN_INIT = 0, FIN_CHECK = 1 };
 
-// totals of the G workgroups' partials (row-major part[b * NR + r], summed in a fixed order), then
-// the scalar stage.  One workgroup: thread 0 the global scalars, thread k < ns shift k.
+// totals of the G workgroups' partials, then the initial scalars or the check's.  One workgroup: thread 0 the global scalars, thread k < ns shift k.
 template <int NR, int STAGE>
-__global__ __launch_bounds__(kBcgBlock) void k_bcg_fin(const double* __restrict__ part, int G, double* st, int ns,
-                                                       double bound, int first) {
-    __shared__ double sm[kBcgBlock / 64][NR];
-    __shared__ double tot[NR];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, t = threadIdx.x;
-    double acc[NR];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) acc[r] = 0.0;
-    for (int b = t; b < G; b += blockDim.x) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) acc[r] += part[(size_t)b * NR + r];
-    }
-#pragma unroll
-    for (int r = 0; r < NR; ++r) acc[r] = wave_sum(acc[r]);
-    if (lane == 0) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) sm[wv][r] = acc[r];
-    }
-    __syncthreads();
-    if (t < NR) {
-        double s = 0.0;
-        for (int q = 0; q < kBcgBlock / 64; ++q) s += sm[q][t];
-        tot[t] = s;
-    }
-    __syncthreads();
+__global__ __launch_bounds__(kFinBlock) void k_bcg_fin(const double* __restrict__ part, int G, double* st, int ns,
+                                                       double bound) {
+    __shared__ double tot[kFinMax];
+    partial_totals<kFinBlock>(part, G, NR, tot);
+    const int t = threadIdx.x;
     const bool mine = t < ns;
-    const bool active = mine && st[oAct + t] != 0.0;
     if (STAGE == FIN_INIT) {
         // delta = <W0, R>; per shift zeta = zeta_old = beta_k = rho = 1, |s_k| = 1 (:88-97, :124)
         if (t == 0) {
-            st[kDelta] = tot[0];
-            st[kDelta + 1] = tot[1];
+            st2(st + kDelta, dcx{tot[0], tot[1]});
+            st2(st + kDeltaNext, dcx{tot[0], tot[1]});
             st[kBeta] = st[kBeta + 1] = st[kAlpha] = st[kAlpha + 1] = 0.0;
         }
         if (mine) {
@@ -334,82 +420,10 @@ __global__ __launch_bounds__(kBcgBlock) void k_bcg_fin(const double* __restrict_
             c[0] = 1.0;
             c[1] = c[2] = c[3] = 0.0;
         }
-    } else if (STAGE == FIN_PHI) {
-        // phi = <W0, SA> / delta (:218); the next step's newbeta = -1 / phi and per-shift zeta, beta_k
-        // (:133-164), then beta = newbeta
-        const dcx phi = cdiv(dcx{tot[0], tot[1]}, ld2(st + kDelta));
-        const dcx nb = cdiv(dcx{-1.0, 0.0}, phi);
-        if (active) {
-            const dcx cn = ld2(st + oCn + 2 * t);
-            const dcx one_cnb = csub(dcx{1.0, 0.0}, cmul(cn, nb));
-            if (first) {
-                const dcx z = cdiv(dcx{1.0, 0.0}, one_cnb);
-                st2(st + oZeta + 2 * t, z);
-                st2(st + oBetas + 2 * t, cmul(nb, z));
-            } else {
-                const dcx beta = ld2(st + kBeta), alpha = ld2(st + kAlpha);
-                const dcx znm1 = ld2(st + oZold + 2 * t);
-                const dcx zold = ld2(st + oZeta + 2 * t);
-                const dcx zb = cmul(znm1, beta);
-                const dcx z = cdiv(cmul(zold, zb), cadd(cmul(alpha, cmul(nb, csub(znm1, zold))), cmul(zb, one_cnb)));
-                st2(st + oZold + 2 * t, zold);
-                st2(st + oZeta + 2 * t, z);
-                st2(st + oBetas + 2 * t, cdiv(cmul(nb, z), zold));
-            }
-        }
-        __syncthreads();  // every shift has read beta
-        if (t == 0) {
-            st2(st + kPhi, phi);
-            st2(st + kBeta, nb);
-        }
-    } else if (STAGE == FIN_CHI) {
-        // chi = <WA, W> / |WA|^2 (:170); per shift (:178-189)
-        const dcx chi = {tot[0] / tot[2], tot[1] / tot[2]};
-        if (t == 0) st2(st + kChi, chi);
-        if (active) {
-            const dcx cn = ld2(st + oCn + 2 * t);
-            const dcx dinom = cadd(dcx{1.0, 0.0}, cmul(cn, chi));
-            const dcx chis = cdiv(chi, dinom);
-            const dcx rho = ld2(st + oRho + 2 * t);
-            const dcx betas = ld2(st + oBetas + 2 * t);
-            const dcx chirho = cmul(chis, rho);
-            const dcx crz = cmul(chirho, ld2(st + oZeta + 2 * t));
-            const dcx crzb = cdiv(crz, betas);
-            const dcx crzob = cdiv(cmul(chirho, ld2(st + oZold + 2 * t)), betas);
-            double* c = st + oC8 + 8 * t;
-            c[0] = -betas.x;
-            c[1] = -betas.y;
-            c[2] = crz.x;
-            c[3] = crz.y;
-            c[4] = -crzb.x;
-            c[5] = -crzb.y;
-            c[6] = crzob.x;
-            c[7] = crzob.y;
-            st2(st + oRho + 2 * t, cdiv(rho, dinom));
-        }
-    } else if (STAGE == FIN_ALPHA) {
-        // delta' = <W0, R>, alpha = beta (-delta') / (chi delta), delta = delta' (:194-196); per shift (:205-209)
-        const dcx nd = {tot[0], tot[1]};
-        const dcx beta = ld2(st + kBeta), chi = ld2(st + kChi);
-        const dcx alpha = cdiv(cmul(beta, dcx{-nd.x, -nd.y}), cmul(chi, ld2(st + kDelta)));
-        if (active) {
-            const dcx z = ld2(st + oZeta + 2 * t);
-            const dcx as = cdiv(cmul(cmul(alpha, z), ld2(st + oBetas + 2 * t)), cmul(ld2(st + oZold + 2 * t), beta));
-            const dcx zr = cmul(z, ld2(st + oRho + 2 * t));
-            double* c = st + oC4 + 4 * t;
-            c[0] = as.x;
-            c[1] = as.y;
-            c[2] = zr.x;
-            c[3] = zr.y;
-        }
-        __syncthreads();  // every shift has read delta
-        if (t == 0) {
-            st2(st + kAlpha, alpha);
-            st2(st + kDelta, nd);
-        }
     } else {
         // the check (:220-242): |S| and the active shifts' |s_k|; a shift below the bound leaves the set
         __shared__ double mx[kBcgMaxShift + 1];
+        const bool active = mine && st[oAct + t] != 0.0;
         if (t <= kBcgMaxShift) mx[t] = 0.0;
         __syncthreads();
         if (active) {
@@ -437,7 +451,7 @@ struct BcgRun {
     int ns;
     BcgShifts sp;
     double* st;
-    double* part;
+    double *part, *pphi, *pchi, *palpha;  // partials: the check's, and each scalar stage's
     double bound;
     int kind, op;
     const clg_field_s* gauge;
@@ -452,28 +466,26 @@ struct BcgRun {
         return linop_apply(ctx, kind, op, gauge, param, out, in);
     }
     template <int NR, int STAGE>
-    void fin(int first = 0) {
-        k_bcg_fin<NR, STAGE><<<1, kBcgBlock, 0, ctx->stream>>>(part, (int)G, st, ns, bound, first);
+    void fin(const double* p) {
+        k_bcg_fin<NR, STAGE><<<1, kFinBlock, 0, ctx->stream>>>(p, (int)G, st, ns, bound);
     }
     // one step of the recurrences: launches only
-    int step() {
+    int step(bool first) {
         hipStream_t s = ctx->stream;
-        k_bcg_w<P><<<G, kBcgBlock, 0, s>>>(n, st, c(R), c(SA), m(W));
+        const int g = (int)G;
+        k_bcg_w<P><<<G, kBcgBlock, 0, s>>>(n, ns, st, pphi, g, first ? 1 : 0, c(R), c(SA), m(W));
         CLG_TRY(apply(WA, W));
-        k_bcg_dot<P, true><<<G, kBcgBlock, 0, s>>>(n, c(WA), c(W), part);
-        fin<3, FIN_CHI>();
-        k_bcg_upd1<P><<<G, kBcgBlock, 0, s>>>(n, ns, sp, st, c(W), c(WA), c(W0), m(R), part);
-        fin<2, FIN_ALPHA>();
-        k_bcg_upd2<P><<<G, kBcgBlock, 0, s>>>(n, st, c(R), c(SA), m(S));
+        k_bcg_dot<P, true><<<G, kBcgBlock, 0, s>>>(n, c(WA), c(W), pchi);
+        k_bcg_upd1<P><<<G, kBcgBlock, 0, s>>>(n, ns, sp, st, pchi, g, c(W), c(WA), c(W0), m(R), palpha);
+        k_bcg_upd2<P><<<G, kBcgBlock, 0, s>>>(n, ns, st, palpha, g, c(R), c(SA), m(S));
         CLG_TRY(apply(SA, S));
-        k_bcg_dot<P, false><<<G, kBcgBlock, 0, s>>>(n, c(W0), c(SA), part);
-        fin<2, FIN_PHI>(0);
+        k_bcg_dot<P, false><<<G, kBcgBlock, 0, s>>>(n, c(W0), c(SA), pphi);
         CLG_HIP(hipGetLastError());
         return CLG_OK;
     }
     int check(double& maxerr, bool& done) {
         k_bcg_norms<P><<<G, kBcgBlock, 0, ctx->stream>>>(n, ns, sp, st, c(S), c(R), part);
-        fin<kBcgNormRows, FIN_CHECK>();
+        fin<kBcgNormRows, FIN_CHECK>(part);
         CLG_HIP(hipGetLastError());
         double h[2];
         CLG_TRY(fetch_doubles(ctx, st + kMaxErr, 2, h));
@@ -516,7 +528,7 @@ int msbicgstab_dev(clg_context ctx, int kind, int op, const clg_field_s* gauge, 
     double* st = nullptr;
     CLG_TRY(workspace(ctx, kBcgState, &st));
     const unsigned G = (unsigned)std::max<long>(1, std::min<long>((n + kBcgBlock - 1) / kBcgBlock, kBcgMaxGrid));
-    CLG_TRY(ensure_reduction_scratch(ctx, (size_t)kBcgMaxGrid * kBcgNormRows));
+    CLG_TRY(ensure_reduction_scratch(ctx, (size_t)kBcgMaxGrid * (kBcgNormRows + 7)));
 
     auto run = [&](auto tag) -> int {
         constexpr int P = decltype(tag)::value;
@@ -531,6 +543,9 @@ int msbicgstab_dev(clg_context ctx, int kind, int op, const clg_field_s* gauge, 
         }
         r.st = st;
         r.part = ctx->red_partial;
+        r.pphi = r.part + (size_t)kBcgMaxGrid * kBcgNormRows;
+        r.pchi = r.pphi + (size_t)kBcgMaxGrid * 2;
+        r.palpha = r.pchi + (size_t)kBcgMaxGrid * 3;
         r.bound = accuracy * blen;
         r.kind = kind;
         r.op = op;
@@ -552,17 +567,20 @@ int msbicgstab_dev(clg_context ctx, int kind, int op, const clg_field_s* gauge, 
         CLG_TRY(blas_axpby(ctx, S, 1.0, 0.0, b, 0.0, 0.0));
         CLG_TRY(blas_conj(ctx, W0, b));
         CLG_HIP(hipMemcpyAsync(st + oCn, shifts.data(), sizeof(double) * 2 * ns, hipMemcpyHostToDevice, s));
-        // delta = <W0, R>; SA = A S; phi = <W0, SA> / delta and the first step's zeta, beta_k (:124-126)
+        // delta = <W0, R>; SA = A S; the partials of the first step's phi (:124-126)
         k_bcg_dot<P, false><<<G, kBcgBlock, 0, s>>>(n, r.c(W0), r.c(R), r.part);
-        r.template fin<2, FIN_INIT>();
+        r.template fin<2, FIN_INIT>(r.part);
         CLG_TRY(r.apply(SA, S));
-        k_bcg_dot<P, false><<<G, kBcgBlock, 0, s>>>(n, r.c(W0), r.c(SA), r.part);
-        r.template fin<2, FIN_PHI>(1);
+        k_bcg_dot<P, false><<<r.G, kBcgBlock, 0, s>>>(n, r.c(W0), r.c(SA), r.pphi);
         CLG_HIP(hipGetLastError());
         // the steps between two checks launch the same work every time: after the first group, which
         // runs directly (operator tuning, scratch growth), they replay as one recorded graph
+        bool first = true;
         auto group = [&]() -> int {
-            for (int i = 0; i < dev_check; ++i) CLG_TRY(r.step());
+            for (int i = 0; i < dev_check; ++i) {
+                CLG_TRY(r.step(first));
+                first = false;
+            }
             return CLG_OK;
         };
         std::vector<unsigned long long> key = {0x4d534243ULL, (unsigned long long)kind, (unsigned long long)op,
