@@ -1021,12 +1021,12 @@ __global__ __launch_bounds__(kFinBlock) void k_bgs_finish(Act act, const double*
         double c2 = 0;
         for (int k = 0; k < 2 * K; ++k) c2 += tot[k] * tot[k];
         double f2 = flag ? w2 - c2 : w2;
-        if (!(f2 > 1e-300)) f2 = 1e-300;
-        const double f = sqrt(f2);
+        const bool none = f2 <= 1e-300;  // an invariant subspace: a zero vector, as in the single-system step
+        const double f = none ? 0.0 : sqrt(f2);
         hcol[2 * (j + 1)] = -f;
         hcol[2 * (j + 1) + 1] = 0.0;
         gs[1] = f2;
-        gs[2] = 1.0 / f;
+        gs[2] = none ? 0.0 : 1.0 / f;
         gs[3] = flag ? 1.0 : 0.0;
     }
 }

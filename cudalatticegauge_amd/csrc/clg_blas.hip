@@ -373,20 +373,6 @@ __global__ __launch_bounds__(256) void k_vmm(VmmArgs a, const double* __restrict
 }
 
 // ---- Hessenberg column of one Gram-Schmidt step (one workgroup); the fast form's and the general one's
-// the column of the fast form from the projections h
-template <int K>
-__device__ __forceinline__ void gs_fast_column(const double* h, double w2, double* hcol, int j, int shifted) {
-    const int i = threadIdx.x;
-    if (i < K) {
-        hcol[2 * i] = shifted ? (i == j ? 1.0 : 0.0) - h[2 * i] : h[2 * i];
-        hcol[2 * i + 1] = shifted ? -h[2 * i + 1] : h[2 * i + 1];
-    }
-    if (i == 0) {
-        const double f = sqrt(w2);
-        hcol[2 * (j + 1)] = shifted ? -f : f;
-        hcol[2 * (j + 1) + 1] = 0.0;
-    }
-}
 // the column from h (hcol) and the second-pass totals
 template <int K>
 __device__ __forceinline__ void gs_slow_column(const double* tot, double* hcol, int j, int shifted, double* sc) {
@@ -412,13 +398,41 @@ __device__ __forceinline__ void gs_slow_column(const double* tot, double* hcol, 
         double c2 = 0;
         for (int k = 0; k < 2 * K; ++k) c2 += tot[k] * tot[k];
         double f2 = flag ? w2 - c2 : w2;
-        if (!(f2 > 1e-300)) f2 = 1e-300;
-        const double f = sqrt(f2);
+        // w lies in the span (its norm is below the rounding of the subtraction): an invariant subspace.  The next
+        // vector is zero, not the noise divided by a tiny norm; NaN stays NaN
+        const bool none = f2 <= 1e-300;
+        const double f = none ? 0.0 : sqrt(f2);
         hcol[2 * (j + 1)] = shifted ? -f : f;
         hcol[2 * (j + 1) + 1] = 0.0;
         sc[1] = f2;
-        sc[2] = 1.0 / f;
+        sc[2] = none ? 0.0 : 1.0 / f;
         sc[3] = flag ? 1.0 : 0.0;
+    }
+}
+// vnext = (w - sum_k h_k V_k) inv
+template <int P, int K>
+__device__ __forceinline__ void gs_sub_scale(long n, const Ptrs<P>& V, const double* hr, const double* hi, double inv,
+                                             const typename Pk<P>::T* w, typename Pk<P>::T* vnext) {
+    constexpr int NC = Pk<P>::NC;
+    GRID_STRIDE(i, n) {
+        typename Pk<P>::T raw[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) raw[k] = V.p[k][i];
+        double y[2 * NC];
+        Pk<P>::ld(w, i, y);
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            double x[2 * NC];
+            Pk<P>::cvt(raw[k], x);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                y[2 * c] -= hr[k] * x[2 * c] - hi[k] * x[2 * c + 1];
+                y[2 * c + 1] -= hr[k] * x[2 * c + 1] + hi[k] * x[2 * c];
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 2 * NC; ++c) y[c] *= inv;
+        Pk<P>::st(vnext, i, y);
     }
 }
 // ---- fused Gram-Schmidt step of the Arnoldi process (see blas_gs_step)
@@ -466,26 +480,7 @@ __global__ __launch_bounds__(kRedBlock) void k_gs_project(long n, Ptrs<P> V, dou
             if (fast && blockIdx.x == 0) gs_fast_column<K>(tot, b2, hcol, j, shifted);
         if (fast) {
             const double inv = 1.0 / sqrt(b2);
-            GRID_STRIDE(i, n) {
-                typename Pk<P>::T raw[K];
-#pragma unroll
-                for (int k = 0; k < K; ++k) raw[k] = V.p[k][i];
-                double y[2 * NC];
-                Pk<P>::ld(w, i, y);
-#pragma unroll
-                for (int k = 0; k < K; ++k) {
-                    double x[2 * NC];
-                    Pk<P>::cvt(raw[k], x);
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) {
-                        y[2 * c] -= hr[k] * x[2 * c] - hi[k] * x[2 * c + 1];
-                        y[2 * c + 1] -= hr[k] * x[2 * c + 1] + hi[k] * x[2 * c];
-                    }
-                }
-#pragma unroll
-                for (int c = 0; c < 2 * NC; ++c) y[c] *= inv;
-                Pk<P>::st(vnext, i, y);
-            }
+            gs_sub_scale<P, K>(n, V, hr, hi, inv, w, vnext);
             return;
         }
     }
@@ -569,7 +564,7 @@ __global__ __launch_bounds__(kRedBlock) void k_gs_finalize(long n, Ptrs<P> V, co
         double f2 = w2;
         if (flag)
             for (int k = 0; k < 2 * K; ++k) f2 -= tot[k] * tot[k];
-        inv = 1.0 / sqrt(f2 > 1e-300 ? f2 : 1e-300);
+        inv = f2 <= 1e-300 ? 0.0 : 1.0 / sqrt(f2);
         if (blockIdx.x == 0) gs_slow_column<K>(tot, hcol, j, shifted, sc);
     } else {
         flag = sc[3] != 0.0;
@@ -610,9 +605,39 @@ __global__ __launch_bounds__(kRedBlock) void k_gs_finalize(long n, Ptrs<P> V, co
     }
 }
 
+// ---- the fast form alone (see blas_gs_fast_step): one pass after the projections, on the shifted operator
+// MERGED: h and |w|^2 are the totals of the projection pass's nin partials, else sc[kGsH..] and sc[0]
+template <int P, int K, bool MERGED>
+__global__ __launch_bounds__(kRedBlock) void k_gs_fast(long n, Ptrs<P> V, const typename Pk<P>::T* __restrict__ w,
+                                                       typename Pk<P>::T* __restrict__ vnext, double* hcol, int j,
+                                                       double* sc, const double* __restrict__ pin, int nin) {
+    __shared__ double tot[MERGED ? kFinMax : 1];
+    const double* h = sc + kGsH;
+    double w2;
+    if constexpr (MERGED) {
+        partial_totals<kRedBlock>(pin, nin, 2 * K + 1, tot);
+        h = tot;
+        w2 = tot[2 * K];
+    } else {
+        w2 = sc[0];
+    }
+    const double inv = gs_fast_scalars<K>(h, w2, hcol, j, sc);
+    double hr[K], hi[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) { hr[k] = h[2 * k]; hi[k] = h[2 * k + 1]; }
+    gs_sub_scale<P, K>(n, V, hr, hi, inv, w, vnext);
+}
+// the cycle's last step needs no vector, only the column: one workgroup
+template <int K>
+__global__ __launch_bounds__(kFinBlock) void k_gs_fast_last(const double* __restrict__ pin, int nin, double* hcol, int j,
+                                                            double* sc) {
+    __shared__ double tot[kFinMax];
+    partial_totals<kFinBlock>(pin, nin, 2 * K + 1, tot);
+    (void)gs_fast_scalars<K>(tot, tot[2 * K], hcol, j, sc);
+}
+
 // workgroups of a reduction: four packets a lane, but one a lane while that gives at most kMergeGrid workgroups (a
 // small vector's pass is a chain of latencies: 12-vector multi-dot at 8^4 7.9 -> 4.4 us)
-constexpr long kMergeGrid = 256;
 unsigned red_grid(clg_context ctx, long n) {
     const long one = (n + kRedBlock - 1) / kRedBlock, four = (one + 3) / 4;
     const long cap = std::min<long>(kMaxRedGrid, (long)ctx->num_cu * 4);
@@ -634,6 +659,8 @@ int h16_norm2_dev(clg_context, const clg_field_s*, double*);
 int h16_scale_inv_sqrt(clg_context, clg_field_s*, const clg_field_s*, const double*);
 int h16_multiaxpy(clg_context, clg_field_s*, clg_field_s* const*, int, const double*, double);
 int h16_gs_step(clg_context, clg_field_s* const*, int, clg_field_s*, double*, int, bool, clg_field_s*, double*);
+int h16_gs_fast_step(clg_context, clg_field_s* const*, int, clg_field_s*, double*, int, clg_field_s*, double*);
+int gs_fast_last(clg_context, unsigned, int, double*, int, double*);
 
 // ---- first-stage buffer of clg_multidot_noalloc: a file-scope device array, so that entry point
 // allocates nothing.  Each device holds its own copy for the life of the process; host code reaches it
@@ -1057,6 +1084,60 @@ int blas_gs_step(clg_context ctx, clg_field_s* const* V, int nv, clg_field_s* w,
     if (pk == PK_D) return gs_step_p<PK_D>(ctx, V, nv, w, hcol, j, shifted, vnext, sc, n);
     if (pk == PK_F4) return gs_step_p<PK_F4>(ctx, V, nv, w, hcol, j, shifted, vnext, sc, n);
     return gs_step_p<PK_F2>(ctx, V, nv, w, hcol, j, shifted, vnext, sc, n);
+}
+
+// One Arnoldi orthogonalisation on a shifted operator (K = 1 - A, whose projections cancel next to nothing) in the
+// fast form of blas_gs_step and without its alternatives: projections, then V_{j+1} and the column in one pass --
+// no finish, no normalisation pass, and no vector pass at all for the last step of a cycle (vnext null).  A step
+// whose |w|^2 - |h|^2 keeps less than half of |w|^2 sets sc[kGsBad] and leaves a zero vector: the caller discards
+// the cycle and repeats it with blas_gs_step.
+template <int P>
+static int gs_fast_p(clg_context ctx, clg_field_s* const* V, int nv, const clg_field_s* w, double* hcol, int j,
+                     clg_field_s* vnext, double* sc, long n) {
+    const unsigned g = red_grid(ctx, n);
+    Ptrs<P> Pp;
+    for (int k = 0; k < nv; ++k) Pp.p[k] = (const typename Pk<P>::T*)V[k]->data;
+    const typename Pk<P>::T* wc = (const typename Pk<P>::T*)w->data;
+#define CALL(KK) k_multidot<P, KK, true><<<g, kRedBlock, 0, ctx->stream>>>(n, Pp, wc, ctx->red_partial, nullptr);
+    SWITCH_K(nv, CALL)
+#undef CALL
+    CLG_HIP(hipGetLastError());
+    if (!vnext) return gs_fast_last(ctx, g, nv, hcol, j, sc);
+    typename Pk<P>::T* vp = (typename Pk<P>::T*)vnext->data;
+    const bool merged = g <= kMergeGrid;
+    if (!merged) CLG_TRY(red_finish(ctx, g, 2 * nv + 1, sc + kGsH, 2 * nv, sc, nullptr, nullptr, 0.0, nullptr));
+#define CALL(KK)                                                                                                        \
+    if (merged)                                                                                                         \
+        k_gs_fast<P, KK, true><<<g, kRedBlock, 0, ctx->stream>>>(n, Pp, wc, vp, hcol, j, sc, ctx->red_partial, (int)g);  \
+    else                                                                                                                \
+        k_gs_fast<P, KK, false><<<g, kRedBlock, 0, ctx->stream>>>(n, Pp, wc, vp, hcol, j, sc, nullptr, 0);
+    SWITCH_K(nv, CALL)
+#undef CALL
+    CLG_HIP(hipGetLastError());
+    return CLG_OK;
+}
+
+// the column of a cycle's last step from g rows of partials in ctx->red_partial
+int gs_fast_last(clg_context ctx, unsigned g, int nv, double* hcol, int j, double* sc) {
+#define CALL(KK) k_gs_fast_last<KK><<<1, kFinBlock, 0, ctx->stream>>>(ctx->red_partial, (int)g, hcol, j, sc);
+    SWITCH_K(nv, CALL)
+#undef CALL
+    CLG_HIP(hipGetLastError());
+    return CLG_OK;
+}
+
+int blas_gs_fast_step(clg_context ctx, clg_field_s* const* V, int nv, clg_field_s* w, double* hcol, int j,
+                      clg_field_s* vnext, double* sc) {
+    CLG_CHECK_ARG(nv >= 1 && nv <= kMaxK, "fused Gram-Schmidt takes 1..%d vectors", kMaxK);
+    if (w && w->prec == CLG_F16) return h16_gs_fast_step(ctx, V, nv, w, hcol, j, vnext, sc);
+    for (int k = 0; k < nv; ++k) CLG_TRY(check_pair(V[k], w));
+    if (vnext) CLG_TRY(check_pair(vnext, w));
+    CLG_TRY(ensure_reduction_scratch(ctx, (size_t)kMaxRedGrid * (2 * kMaxK + 1)));
+    long n;
+    const int pk = pk_of(w, n);
+    if (pk == PK_D) return gs_fast_p<PK_D>(ctx, V, nv, w, hcol, j, vnext, sc, n);
+    if (pk == PK_F4) return gs_fast_p<PK_F4>(ctx, V, nv, w, hcol, j, vnext, sc, n);
+    return gs_fast_p<PK_F2>(ctx, V, nv, w, hcol, j, vnext, sc, n);
 }
 
 // copies `count` doubles from device to the context's pinned buffer and waits

@@ -22,6 +22,7 @@ using namespace clgd;
 namespace clg {
 int red_finish_partials(clg_context, unsigned, int, double*, int, double*, const int*, const double*, double, int*);
 int gs_finish_launch(clg_context, unsigned, int, double*, int, bool, double*, bool);
+int gs_fast_last(clg_context, unsigned, int, double*, int, double*);
 int ensure_reduction_scratch(clg_context, size_t);
 }  // namespace clg
 
@@ -132,6 +133,41 @@ __global__ __launch_bounds__(kRedBlock) void k_h_multidot(unsigned n, unsigned V
     block_partial<2 * K + 1>(acc, partial);
 }
 
+// (oc, os) = (w - sum_k h_k V_k) inv
+template <int K>
+__device__ __forceinline__ void h_gs_sub_scale(unsigned n, unsigned Vh, const HTab& V, const float* hr, const float* hi,
+                                               float inv, const uint4* wc, const float* ws, uint4* oc, float* os) {
+    SITE_LOOP(i, n) {
+        float sv[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) sv[k] = V.v[k].s[i];
+        const float sw = ws[i];
+        float y[24];
+#pragma unroll
+        for (int ch = 0; ch < 3; ++ch) {
+            const size_t ci = h16_chunk(i, Vh, ch);
+            uint4 raw[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) raw[k] = V.v[k].c[ci];
+            float* yc = y + 8 * ch;
+            h16_unpack8(wc[ci], sw, yc);
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                float x[8];
+                h16_unpack8(raw[k], sv[k], x);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    yc[2 * q] -= hr[k] * x[2 * q] - hi[k] * x[2 * q + 1];
+                    yc[2 * q + 1] -= hr[k] * x[2 * q + 1] + hi[k] * x[2 * q];
+                }
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 24; ++q) y[q] *= inv;
+        h16_store_site(oc, os, Vh, i, y);
+    }
+}
+
 // w' = w - sum_k h_k V_k, stored to (oc, os) (w itself or the next basis vector), with the
 // partials of V_k^H w' and |w'|^2 of the unrounded w'.  fast_ok (oc is the next basis vector): the
 // fast form of the FP64 / FP32 step (k_gs_project) -- when |w|^2 - |h|^2 keeps half of |w|^2, w'/|w'|
@@ -158,35 +194,7 @@ __global__ __launch_bounds__(kRedBlock) void k_h_gs_project(unsigned n, unsigned
         }
         if (fast) {
             const float inv = (float)(1.0 / sqrt(b2));
-            SITE_LOOP(i, n) {
-                float sv[K];
-#pragma unroll
-                for (int k = 0; k < K; ++k) sv[k] = V.v[k].s[i];
-                const float sw = ws[i];
-                float y[24];
-#pragma unroll
-                for (int ch = 0; ch < 3; ++ch) {
-                    const size_t ci = h16_chunk(i, Vh, ch);
-                    uint4 raw[K];
-#pragma unroll
-                    for (int k = 0; k < K; ++k) raw[k] = V.v[k].c[ci];
-                    float* yc = y + 8 * ch;
-                    h16_unpack8(wc[ci], sw, yc);
-#pragma unroll
-                    for (int k = 0; k < K; ++k) {
-                        float x[8];
-                        h16_unpack8(raw[k], sv[k], x);
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            yc[2 * q] -= hr[k] * x[2 * q] - hi[k] * x[2 * q + 1];
-                            yc[2 * q + 1] -= hr[k] * x[2 * q + 1] + hi[k] * x[2 * q];
-                        }
-                    }
-                }
-#pragma unroll
-                for (int q = 0; q < 24; ++q) y[q] *= inv;
-                h16_store_site(oc, os, Vh, i, y);
-            }
+            h_gs_sub_scale<K>(n, Vh, V, hr, hi, inv, wc, ws, oc, os);
             return;
         }
     }
@@ -239,6 +247,28 @@ __global__ __launch_bounds__(kRedBlock) void k_h_gs_project(unsigned n, unsigned
         acc[2 * K] += ww;
     }
     block_partial<2 * K + 1>(acc, partial);
+}
+
+// the fast form alone (k_gs_fast of the FP64 / FP32 step), the scalars as there
+template <int K, bool MERGED>
+__global__ __launch_bounds__(kRedBlock) void k_h_gs_fast(unsigned n, unsigned Vh, HTab V, const uint4* wc, const float* ws,
+                                                         uint4* oc, float* os, double* hcol, int j, double* sc,
+                                                         const double* __restrict__ pin, int nin) {
+    __shared__ double tot[MERGED ? kFinMax : 1];
+    const double* h = sc + kGsH;
+    double w2;
+    if constexpr (MERGED) {
+        partial_totals<kRedBlock>(pin, nin, 2 * K + 1, tot);
+        h = tot;
+        w2 = tot[2 * K];
+    } else {
+        w2 = sc[0];
+    }
+    const float inv = (float)gs_fast_scalars<K>(h, w2, hcol, j, sc);
+    float hr[K], hi[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) { hr[k] = (float)h[2 * k]; hi[k] = (float)h[2 * k + 1]; }
+    h_gs_sub_scale<K>(n, Vh, V, hr, hi, inv, wc, ws, oc, os);
 }
 
 // in place on vnext, which holds w': vnext = (w' - flag sum_k c2_k V_k) / |w''| (sc as written by
@@ -441,6 +471,36 @@ int h16_gs_step(clg_context ctx, clg_field_s* const* V, int nv, clg_field_s* w, 
 #undef CALL
         CLG_HIP(hipGetLastError());
     }
+    return CLG_OK;
+}
+
+// the FP16 form of blas_gs_fast_step
+int h16_gs_fast_step(clg_context ctx, clg_field_s* const* V, int nv, clg_field_s* w, double* hcol, int j,
+                     clg_field_s* vnext, double* sc) {
+    HTab t;
+    CLG_TRY(table(V, nv, w, t));
+    if (vnext) CLG_TRY(check16(vnext, w));
+    CLG_TRY(ensure_reduction_scratch(ctx, (size_t)kMaxGrid * (2 * kMaxV + 1)));
+    const unsigned n = nsites(w), g = red_grid16(ctx, n), Vh = (unsigned)w->Vh;
+#define CALL(KK) k_h_multidot<KK><<<g, kRedBlock, 0, ctx->stream>>>(n, Vh, t, hptr(w), ctx->red_partial);
+    SWITCH_V(nv, CALL)
+#undef CALL
+    CLG_HIP(hipGetLastError());
+    if (!vnext) return gs_fast_last(ctx, g, nv, hcol, j, sc);
+    const bool merged = g <= (unsigned)kMergeGrid;
+    if (!merged)
+        CLG_TRY(red_finish_partials(ctx, g, 2 * nv + 1, sc + kGsH, 2 * nv, sc, nullptr, nullptr, 0.0, nullptr));
+#define CALL(KK)                                                                                                         \
+    if (merged)                                                                                                          \
+        k_h_gs_fast<KK, true><<<g, kRedBlock, 0, ctx->stream>>>(n, Vh, t, (const uint4*)w->data, w->norm,                 \
+                                                                (uint4*)vnext->data, vnext->norm, hcol, j, sc,            \
+                                                                ctx->red_partial, (int)g);                                \
+    else                                                                                                                 \
+        k_h_gs_fast<KK, false><<<g, kRedBlock, 0, ctx->stream>>>(n, Vh, t, (const uint4*)w->data, w->norm,                \
+                                                                 (uint4*)vnext->data, vnext->norm, hcol, j, sc, nullptr, 0);
+    SWITCH_V(nv, CALL)
+#undef CALL
+    CLG_HIP(hipGetLastError());
     return CLG_OK;
 }
 

@@ -172,6 +172,10 @@ int reduction_ready(clg_context ctx);
 int noalloc_scratch_init(int device);
 // device scratch (doubles) one Arnoldi orthogonalisation step (arn_step, clg_arnoldi.hip) needs
 constexpr int kArnScratch = 264;
+// up to this many workgroups of partials the pass after a small reduction totals them itself
+constexpr long kMergeGrid = 256;
+// within that scratch, of the fast Gram-Schmidt steps: whether one was refused, and the projections
+constexpr int kGsBad = 39, kGsH = 40;
 // scratch field of the same shape as `like` (kind/prec/subset/dims), index slot
 int scratch_field(clg_context ctx, const clg_field_s* like, int kind, int prec, int subset,
                   int slot, clg_field_s** out);
@@ -1142,12 +1146,14 @@ __device__ __forceinline__ void partial_totals(const double* __restrict__ partia
 // Least-squares solution of the (m+1) x m Hessenberg system H y = sqrt(beta2) e_1 by one wave (m <= 64): Givens
 // rotations and back substitution as RotateH / SolveY (CSolverGMRES.cpp:262-358), FP64.  H is column-major with
 // leading dimension ld; sm holds m * ld complex numbers of LDS.  Lane j carries column j: a rotation is one
-// broadcast and four products a lane, and the back substitution eliminates column by column.  dev[0] = |g_m|^2,
+// broadcast and four products a lane, and the back substitution eliminates column by column.  A column of
+// zeros (the vectors after an invariant subspace) gets y = 0.  dev[0] = |g_m|^2,
 // dev[1] = |g_m|.  Measured for m = 12: 7.7 us (one thread on
 // global memory: 28).
 __device__ __forceinline__ cd lane_bcast(cd a, int src) { return cd{__shfl(a.x, src, 64), __shfl(a.y, src, 64)}; }
+// With *bad set (a refused fast Gram-Schmidt step in the cycle) y is zero; dev[2] passes it on.
 __device__ __forceinline__ void gmres_lsq_wave(const double* __restrict__ H, int ld, int m, double beta2, double* y,
-                                               double* dev, cd* sm) {
+                                               double* dev, cd* sm, const double* bad = nullptr) {
     const int lane = (int)(threadIdx.x & 63), col = min(lane, m - 1);
     for (int i = lane; i < m * ld; i += 64) sm[i] = cd{H[2 * i], H[2 * i + 1]};
     __syncthreads();
@@ -1155,8 +1161,9 @@ __device__ __forceinline__ void gmres_lsq_wave(const double* __restrict__ H, int
     for (int k = 0; k < m; ++k) {
         const cd nxt = sm[col * ld + k + 1];  // below the subdiagonal of columns < k: not used
         const cd hkk = lane_bcast(cur, k), hk1 = lane_bcast(nxt, k);
-        const double den = 1.0 / sqrt(hkk.x * hkk.x + hkk.y * hkk.y + hk1.x * hk1.x + hk1.y * hk1.y);
-        const cd cs = cscale(hkk, den), sn = cscale(hk1, den);
+        const double n2 = hkk.x * hkk.x + hkk.y * hkk.y + hk1.x * hk1.x + hk1.y * hk1.y;
+        const double den = n2 == 0.0 ? 0.0 : 1.0 / sqrt(n2);
+        const cd cs = n2 == 0.0 ? cd{1.0, 0.0} : cscale(hkk, den), sn = cscale(hk1, den);
         const cd gk = cmul(cconj(cs), g);
         g = cmul(sn, cd{-g.x, -g.y});
         if (lane == k) z = gk;
@@ -1168,12 +1175,18 @@ __device__ __forceinline__ void gmres_lsq_wave(const double* __restrict__ H, int
     if (lane == 0) {
         dev[0] = g.x * g.x + g.y * g.y;
         dev[1] = sqrt(dev[0]);
+        if (bad) dev[2] = *bad;
+    }
+    if (bad && *bad != 0.0) {
+        if (lane < m) y[2 * lane] = y[2 * lane + 1] = 0.0;
+        return;
     }
     __syncthreads();
     for (int k = m - 1; k >= 0; --k) {
         const cd d = sm[k * ld + k], acc = lane_bcast(z, k);
         const double dd = d.x * d.x + d.y * d.y;
-        const cd yk = cd{(acc.x * d.x + acc.y * d.y) / dd, (acc.y * d.x - acc.x * d.y) / dd};
+        const cd yk = dd == 0.0 ? cd{0.0, 0.0}
+                                : cd{(acc.x * d.x + acc.y * d.y) / dd, (acc.y * d.x - acc.x * d.y) / dd};
         if (lane == k) z = yk;
         else if (lane < k) z = csub(z, cmul(sm[k * ld + lane], yk));
     }
@@ -1181,6 +1194,39 @@ __device__ __forceinline__ void gmres_lsq_wave(const double* __restrict__ H, int
         y[2 * lane] = z.x;
         y[2 * lane + 1] = z.y;
     }
+}
+
+// ---- Gram-Schmidt steps of GMRES: Hessenberg column hcol (column j, interleaved complex) from the projections
+// the column of the fast form from the projections h
+template <int K>
+__device__ __forceinline__ void gs_fast_column(const double* h, double w2, double* hcol, int j, int shifted) {
+    const int i = threadIdx.x;
+    if (i < K) {
+        hcol[2 * i] = shifted ? (i == j ? 1.0 : 0.0) - h[2 * i] : h[2 * i];
+        hcol[2 * i + 1] = shifted ? -h[2 * i + 1] : h[2 * i + 1];
+    }
+    if (i == 0) {
+        const double f = sqrt(w2);
+        hcol[2 * (j + 1)] = shifted ? -f : f;
+        hcol[2 * (j + 1) + 1] = 0.0;
+    }
+}
+// the step's scalars from h and |w|^2: the scale of w' (0 where the fast form does not hold); workgroup 0 writes
+// the column and notes in sc[clg::kGsBad] whether any fast step of the cycle (j = 1 is its first) was refused
+template <int K>
+__device__ __forceinline__ double gs_fast_scalars(const double* h, double w2, double* hcol, int j, double* sc) {
+    double b2 = w2;
+#pragma unroll
+    for (int k = 0; k < 2 * K; ++k) b2 -= h[k] * h[k];
+    const bool ok = b2 >= 0.5 * w2 && b2 > 1e-300;
+    if (blockIdx.x == 0) {
+        gs_fast_column<K>(h, ok ? b2 : 0.0, hcol, j, 1);
+        if (threadIdx.x == 0) {
+            if (!ok) sc[clg::kGsBad] = 1.0;
+            else if (j == 1) sc[clg::kGsBad] = 0.0;
+        }
+    }
+    return ok ? 1.0 / sqrt(b2) : 0.0;
 }
 
 }  // namespace clgd

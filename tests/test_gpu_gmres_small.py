@@ -55,3 +55,26 @@ def test_long_bases(ctx, max_dim):
     st, _ = clg.solve(ctx, p, x, put(ctx, clg.WILSON, clg.F64, dims, b), g, 0.13, clg.EFO_F_D)
     r = orc.wilson_op(dims, orc.BC_FERMION, 0.13, U, x.download()) - b
     assert st == clg.OK and np.linalg.norm(r) < 1.01e-11 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("inner", [clg.F64, clg.F32, clg.INNER_F16_VECTORS])
+@pytest.mark.parametrize("dims", [(4, 4, 4, 4), (16, 16, 16, 16)])
+@pytest.mark.parametrize("noise", [0.0, 1e-12, 1e-3])
+def test_refused_fast_steps(ctx, inner, dims, noise):
+    """On the unit field a constant source spans an invariant subspace of D, and one with some noise nearly so: K V_j
+    lies in the span of the basis after a few steps, the fast Gram-Schmidt step is refused, the cycle repeated in the
+    general form, and a basis that is exhausted ends in zero vectors."""
+    g, b = clg.Field(ctx, clg.GAUGE, clg.F64, dims), clg.Field(ctx, clg.WILSON, clg.F64, dims, bc=(1, 1, 1, 1))
+    g.gauge_unit()
+    src = np.tile(np.arange(1, 25, dtype=float), int(np.prod(dims)))
+    src += noise * np.random.default_rng(1).standard_normal(src.size)
+    b.upload(src)
+    x, r = (clg.Field(ctx, clg.WILSON, clg.F64, dims, bc=(1, 1, 1, 1)) for _ in range(2))
+    for eo in (0, 1):
+        p = clg.solver_params(max_dim=12, restart=50, accuracy=1e-10, stop_rule=clg.STOP_TRUE_RESIDUAL, even_odd=eo,
+                              inner_prec=inner, inner_accuracy=1e-2, max_outer=60)
+        st, rep = clg.solve(ctx, p, x, b, g, 0.11, clg.EFO_F_D)
+        clg.wilson_apply(ctx, r, x, g, 0.11)
+        clg.axpy(ctx, r, -1.0, b)
+        res = np.sqrt(clg.norm2(ctx, r) / clg.norm2(ctx, b))
+        assert st == clg.OK and res < 1e-10, (eo, rep.cycles, rep.true_residual, res)
