@@ -209,17 +209,23 @@ struct HopBatch {
     double a[kMaxSys];
 };
 
+// whether two systems may share a segment: one gauge field, one coefficient, the same boundary signs (the
+// segment's Geo carries them for all its right-hand sides)
+bool same_segment(const HopBatch& B, int i, int k) {
+    return B.gauge[i] == B.gauge[k] && B.a[i] == B.a[k] && std::equal(B.in[i]->bc, B.in[i]->bc + 4, B.in[k]->bc);
+}
+
 // build the kernel arguments for a tile size; returns the padded grid
 int build_args(const HopBatch& B, int nr, int block, int xcd, bool hasx, double br, int pbase, int nblk,
                BHopArgs& a, unsigned& grid) {
     std::memset(&a, 0, sizeof(a));
-    // group systems by (gauge field, coefficient), keeping first-appearance order
+    // group the systems that may share a segment, keeping first-appearance order
     std::vector<int> order;
     std::vector<bool> used(B.n, false);
     for (int i = 0; i < B.n; ++i) {
         if (used[i]) continue;
         for (int k = i; k < B.n; ++k) {
-            if (!used[k] && B.gauge[k] == B.gauge[i] && B.a[k] == B.a[i]) {
+            if (!used[k] && same_segment(B, i, k)) {
                 used[k] = true;
                 order.push_back(k);
             }
@@ -233,9 +239,7 @@ int build_args(const HopBatch& B, int nr, int block, int xcd, bool hasx, double 
     while (i < order.size()) {
         const int s0 = order[i];
         int cnt = 0;
-        while (i + cnt < order.size() && cnt < nr && B.gauge[order[i + cnt]] == B.gauge[s0] &&
-               B.a[order[i + cnt]] == B.a[s0])
-            ++cnt;
+        while (i + cnt < order.size() && cnt < nr && same_segment(B, order[i + cnt], s0)) ++cnt;
         CLG_CHECK_ARG(nseg < kMaxSys, "too many batch segments");
         BSeg& sg = a.seg[nseg++];
         sg.g = make_geo(B.in[s0]);
