@@ -688,14 +688,17 @@ static double* noalloc_scratch(int device) {
     return g_noalloc_ptr[device];
 }
 
+// An outgrown buffer lives until the context ends: a recorded graph keeps the address its reductions were
+// recorded with (a refused energy call leaves its launches in an open recording).  Nothing is freed or waited for,
+// so growth is also possible while recording.  Each buffer is at least twice the one before, so those kept are
+// together smaller than the current one (0.5 to 9 MB in most programs; a multi-dot of 1000 vectors takes 34 MB).
 int ensure_reduction_scratch(clg_context ctx, size_t doubles) {
     if (ctx->red_partial_cap >= doubles) return CLG_OK;
-    if (ctx->red_partial) {
-        CLG_HIP(hipStreamSynchronize(ctx->stream));
-        (void)hipFree(ctx->red_partial);
-        ctx->red_partial = nullptr;
-    }
-    CLG_HIP(hipMalloc((void**)&ctx->red_partial, doubles * sizeof(double)));
+    doubles = std::max(doubles, 2 * ctx->red_partial_cap);
+    double* grown = nullptr;
+    CLG_HIP(hipMalloc((void**)&grown, doubles * sizeof(double)));
+    if (ctx->red_partial) ctx->red_outgrown.push_back(ctx->red_partial);
+    ctx->red_partial = grown;
     ctx->red_partial_cap = doubles;
     return CLG_OK;
 }

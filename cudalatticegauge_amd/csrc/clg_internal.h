@@ -77,6 +77,7 @@ struct clg_context_s {
     // reduction scratch: per-block partials, device results
     double* red_partial = nullptr;
     size_t red_partial_cap = 0;  // doubles
+    std::vector<double*> red_outgrown;  // earlier, smaller ones: recorded graphs may still write to them
     double* red_result = nullptr;  // 4096 doubles of device-resident results
     double* host_result = nullptr;  // pinned
     // solver workspace (Hessenberg, Givens, scalars), grow-only

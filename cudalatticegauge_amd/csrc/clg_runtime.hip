@@ -519,6 +519,7 @@ int clg_finalize(clg_context c) {
     for (clg_field_s* f : c->scratch) clg_field_destroy(f);
     c->scratch.clear();
     if (c->red_partial) (void)hipFree(c->red_partial);
+    for (double* p : c->red_outgrown) (void)hipFree(p);
     if (c->red_result) (void)hipFree(c->red_result);
     if (c->host_result) (void)hipHostFree(c->host_result);
     if (c->ws) (void)hipFree(c->ws);
@@ -542,7 +543,7 @@ int clg_graph_begin(clg_context c) {
     CLG_CHECK_ARG(c, "null context");
     CLG_CHECK_ARG(!stream_capturing(c), "the context already records a graph");
     (void)hipSetDevice(c->device);
-    // recorded reductions keep the partial-sum buffer they were recorded with: allocate it first
+    // recorded reductions keep the partial-sum buffer they were recorded with: allocate the usual one first
     CLG_TRY(reduction_ready(c));
     CLG_HIP(hipStreamSynchronize(c->stream));
     CLG_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeRelaxed));
