@@ -41,7 +41,7 @@ template <int P> struct ArnPtrs {
     const typename Pk<P>::T* p[kArnMaxV];
 };
 
-// scratch layout (doubles): [0] |w|^2, [1] |w''|^2, [2] 1/|w''|, [3] the flag (as an int), [4, 4+128)
+// scratch layout (doubles): [0] |w|^2, [1] |w''|^2, [2] 1/|w''| (0 when w lies in the span), [3] the flag (as an int), [4, 4+128)
 // c2, [132, 132+128) h
 constexpr int kScFlag = 3, kScC2 = 4, kScH = 4 + 2 * kArnMaxV;
 
@@ -190,12 +190,15 @@ __global__ __launch_bounds__(kArnFinBlock) void k_arn_fin(const double* __restri
         hcol[2 * k + 1] = im;
     }
     if (k == 0) {
-        if (!(f2 > 1e-300)) f2 = 1e-300;  // a breakdown (w in the span) still gives a finite column
+        // w in the span: a finite column with a subdiagonal that is negligible but not zero (the shifted solvers
+        // divide by it), and a zero next vector (what is left of w, scaled by 1e150, would overflow two steps on)
+        const bool none = f2 <= 1e-300;
+        if (!(f2 > 1e-300)) f2 = 1e-300;
         const double f = sqrt(f2);
         hcol[2 * (j + 1)] = shifted ? -f : f;
         hcol[2 * (j + 1) + 1] = 0.0;
         sc[1] = f2;
-        sc[2] = 1.0 / f;
+        sc[2] = none ? 0.0 : 1.0 / f;
     }
 }
 

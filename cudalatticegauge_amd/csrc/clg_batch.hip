@@ -512,7 +512,7 @@ __global__ __launch_bounds__(kRedBlock) void k_bnorm2(const BTab* T, Act act, in
     block_partial<1>(acc, partial + (size_t)blockIdx.y * gridDim.x);
 }
 
-// dst = src / sqrt(n2[s * nstride]); cond (nullable): systems with cond[s * nstride] == 0 skip
+// dst = src / sqrt(n2[s * nstride]), zero for a zero src; cond (nullable): systems with cond[s * nstride] == 0 skip
 template <int P>
 __global__ void k_bscale(const BTab* T, Act act, int dsel, int ssel, const double* n2, int nstride,
                          const double* cond = nullptr) {
@@ -521,7 +521,7 @@ __global__ void k_bscale(const BTab* T, Act act, int dsel, int ssel, const doubl
     typedef typename BP<P>::T PT;
     const PT* src = (const PT*)vec_of(T, s, ssel);
     PT* dst = (PT*)vec_of(T, s, dsel);
-    const double f = 1.0 / sqrt(n2[(size_t)s * nstride]);
+    const double v = n2[(size_t)s * nstride], f = v == 0.0 ? 0.0 : 1.0 / sqrt(v);
     const long n = T->npk[s];
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
         double a[2 * BP<P>::NC];
@@ -799,7 +799,8 @@ __global__ __launch_bounds__(kRedBlock) void k_bh_norm2(const BTab* T, Act act, 
 __global__ __launch_bounds__(256) void k_bh_scale(const BTab* T, Act act, int dsel, int ssel, const double* n2, int stride) {
     const int s = act.idx[blockIdx.y];
     const unsigned n = T->vh[s];
-    const float f = (float)(1.0 / sqrt(n2[(size_t)s * stride]));
+    const double v2 = n2[(size_t)s * stride];
+    const float f = v2 == 0.0 ? 0.f : (float)(1.0 / sqrt(v2));
     const uint4* sc = hvec(T, s, ssel);
     const float* sn = hnrm(T, s, ssel);
     uint4* dc = hvec(T, s, dsel);

@@ -81,7 +81,8 @@ __global__ __launch_bounds__(kRedBlock) void k_h_norm2(unsigned n, unsigned Vh, 
 // dst = src / sqrt(nrm2[0])
 __global__ __launch_bounds__(256) void k_h_scale_inv_sqrt(unsigned n, unsigned Vh, const double* __restrict__ nrm2, HPtr src, uint4* dc,
                                    float* ds) {
-    const float f = (float)(1.0 / sqrt(nrm2[0]));
+    const double v2 = nrm2[0];
+    const float f = v2 == 0.0 ? 0.f : (float)(1.0 / sqrt(v2));
     SITE_LOOP(i, n) {
         float v[24];
         h16_load_site(src.c, src.s, Vh, i, v);

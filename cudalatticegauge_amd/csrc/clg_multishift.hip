@@ -355,10 +355,29 @@ int msgmres(clg_context ctx, OpRef& A, std::vector<clg_field_s*>& X, const std::
         // columns hold rows 0..j+1 only; the device entries below the sub-diagonal are stale
         for (int j = 0; j < m; ++j)
             for (int i = 0; i <= j + 1; ++i) Hb(i, j) = zc(hh[2 * (j * ld + i)], hh[2 * (j * ld + i) + 1]);
+        // min_y |g0 e_1 - (H + c) y| over the first mm columns
+        auto lsq = [&](int mm, zc c, zc g0, std::vector<zc>& y) {
+            Mat Hc(mm + 1, mm);
+            for (int j = 0; j < mm; ++j)
+                for (int i = 0; i <= mm && i <= j + 1; ++i) Hc(i, j) = Hb(i, j) + (i == j ? c : zc(0.0, 0.0));
+            std::vector<zc> rhs(mm + 1, zc(0.0, 0.0));
+            rhs[0] = g0;
+            const double res = clg::sla::hessenberg_lsq(Hc, rhs, y);
+            y.resize(m, zc(0.0, 0.0));
+            return res;
+        };
+        // an Arnoldi step that found w in the span leaves a subdiagonal of 1e-150: the space is closed, every
+        // shifted system is solved in it by itself, and there is no common residual direction to keep
+        int mm = m;
+        bool closed = false;
+        for (int j = 0; j < m && !closed; ++j)
+            if (std::abs(Hb(j + 1, j)) < 2e-150) {
+                mm = j + 1;
+                closed = true;
+            }
         // unshifted least squares, x_base += V y, z = beta e_1 - Hbar y
-        std::vector<zc> rhs(m + 1, zc(0.0, 0.0)), y;
-        rhs[0] = beta;
-        clg::sla::hessenberg_lsq(Hb, rhs, y);
+        std::vector<zc> y;
+        lsq(mm, zc(0.0, 0.0), beta, y);
         std::vector<zc> z(m + 1, zc(0.0, 0.0));
         z[0] = beta;
         for (int i = 0; i <= m; ++i)
@@ -368,6 +387,16 @@ int msgmres(clg_context ctx, OpRef& A, std::vector<clg_field_s*>& X, const std::
         // shifted systems
         maxerr = 0;
         for (int n = 0; n < ns; ++n) {
+            if (closed) {
+                std::vector<zc> yc;
+                maxerr = std::max(maxerr, lsq(mm, zc(shifts[n].x, shifts[n].y), beta0[n] * beta, yc));
+                beta0[n] = zc(0.0, 0.0);
+                for (int j = 0; j < m; ++j) {
+                    up[2 * (size_t)m * (n + 1) + 2 * j] = yc[j].real();
+                    up[2 * (size_t)m * (n + 1) + 2 * j + 1] = yc[j].imag();
+                }
+                continue;
+            }
             Mat M(m + 1, m + 1);
             for (int i = 0; i <= m; ++i) {
                 for (int j = 0; j < m; ++j) M(i, j) = Hb(i, j) + (i == j ? zc(shifts[n].x, shifts[n].y) : zc(0.0, 0.0));
@@ -407,6 +436,7 @@ int msgmres(clg_context ctx, OpRef& A, std::vector<clg_field_s*>& X, const std::
         CLG_HIP(hipGetLastError());
         CLG_HIP(hipStreamSynchronize(ctx->stream));  // up is a host temporary
         if (maxerr < accuracy * blen) return CLG_OK;
+        if (closed) return CLG_NOT_CONVERGED;  // a shifted operator that is singular on the space: nothing to restart
     }
     return CLG_NOT_CONVERGED;
 }

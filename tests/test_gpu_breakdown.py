@@ -1,6 +1,6 @@
 """Krylov spaces that close after one vector: on the unit field D acts on a constant spinor field as a number.  The
 basis then ends in zero vectors, whatever the rounding leaves of the next one (nothing, or noise), in the bases of up
-to 64 vectors, the shifted solvers and the batched solver as in the short single-system ones."""
+to 64 vectors, the shifted solvers, the deflated and the batched solver as in the short single-system ones."""
 import numpy as np
 import pytest
 
@@ -88,3 +88,15 @@ def test_shifted(ctx, site, solver):
         # D b = (1 - 8 kappa) b, so x = b / (1/2 + s)
         err = np.abs(x.download() * (0.5 + s) - want).max() / np.abs(want).max()
         assert st == clg.OK and err < 1e-12, (s, err)
+
+
+@pytest.mark.parametrize("site", [EXACT, NOISY])
+@pytest.mark.parametrize("m_dim", [8, 24])
+@pytest.mark.parametrize("deflate", [clg.DEFLATE_REV, clg.DEFLATE_HEV, clg.DEFLATE_SVD])
+def test_deflated(ctx, site, m_dim, deflate):
+    g, b, x = unit(ctx), spinor(ctx, site), empty(ctx)
+    s = clg.Gcrodr(ctx, m_dim=m_dim, k_dim=4, restart=20, accuracy=1e-22, deflate=deflate)
+    st, _ = s.solve(x, b, g, 0.0625, clg.EFO_F_D)
+    res = residual(ctx, x, b, g, 0.0625)
+    s.close()
+    assert st == clg.OK and res < 1e-12, res
