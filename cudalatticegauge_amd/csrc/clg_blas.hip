@@ -443,8 +443,8 @@ __device__ __forceinline__ void gs_sub_scale(long n, const Ptrs<P>& V, const dou
 // applies: w' / |w'| goes straight to vnext and no partials are taken.  Workgroup 0 records the choice
 // in sc ([1] |w'|^2, [2] 1/|w'|, [3] 2 for the fast form, else 0) for the finish and finalize.
 // MERGED (small vectors): h and |w|^2 are not finished yet; every workgroup totals the projection pass's nin
-// partials itself (two launches less per step), workgroup 0 stores h to hcol and |w|^2 to sc[0], and in the fast
-// form also the finished column.
+// partials itself (two launches less per step), workgroup 0 stores |w|^2 to sc[0] and to hcol either the finished
+// column (fast form) or h.
 template <int P, int K, bool MERGED>
 __global__ __launch_bounds__(kRedBlock) void k_gs_project(long n, Ptrs<P> V, double* hcol, typename Pk<P>::T* w, double* partial,
                                                            double* sc, typename Pk<P>::T* vnext,
@@ -455,10 +455,7 @@ __global__ __launch_bounds__(kRedBlock) void k_gs_project(long n, Ptrs<P> V, dou
     if constexpr (MERGED) {
         partial_totals<kRedBlock>(pin, nin, 2 * K + 1, tot);
         h = tot;
-        if (blockIdx.x == 0) {
-            if (threadIdx.x < 2 * K) hcol[threadIdx.x] = tot[threadIdx.x];
-            else if (threadIdx.x == 2 * K) sc[0] = tot[2 * K];
-        }
+        if (blockIdx.x == 0 && threadIdx.x == 0) sc[0] = tot[2 * K];
     }
     double hr[K], hi[K];
 #pragma unroll
@@ -484,6 +481,8 @@ __global__ __launch_bounds__(kRedBlock) void k_gs_project(long n, Ptrs<P> V, dou
             return;
         }
     }
+    if constexpr (MERGED)
+        if (blockIdx.x == 0 && threadIdx.x < 2 * K) hcol[threadIdx.x] = tot[threadIdx.x];
     double v[2 * K + 1];
 #pragma unroll
     for (int k = 0; k < 2 * K + 1; ++k) v[k] = 0;
