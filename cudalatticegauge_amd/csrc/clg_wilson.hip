@@ -458,7 +458,7 @@ bool valid_cfg(int pm, int blk, int xcd, int spt) {
     return pm >= 1 && pm <= 8 && (blk == 64 || blk == 128 || blk == 256) &&
            (xcd == 0 || xcd == 1 || xcd == 8 || tiled_xcd(xcd)) && (spt == 1 || spt == 2 || spt == 4);
 }
-// the configurations in 64-site blocks (the tuner's, its cache file's and CLG_TUNE_FORCE's): the
+// the configurations in 64-site blocks (the tuner's, its cache file's and forced ones): the
 // direction-split kernel, and one site per thread in the tiled order
 bool valid_split(int pm, int blk, int xcd, int spt) {
     if (blk != kSplitSites || spt != 1) return false;
@@ -801,9 +801,10 @@ int clg_autotune_force(int pin_mode, int block, int xcd, int sites_per_thread) {
         return CLG_OK;
     }
     if (sites_per_thread == 0) sites_per_thread = 1;
-    CLG_CHECK_ARG(valid_cfg(pin_mode, block, xcd, sites_per_thread),
+    CLG_CHECK_ARG(valid_cfg(pin_mode, block, xcd, sites_per_thread) || valid_split(pin_mode, block, xcd, sites_per_thread),
                   "pin_mode 1..8, block 64|128|256, xcd 0|1|8 or a tiled plane schedule 20|21|40|41|80|81, "
-                  "sites_per_thread 1|2|4");
+                  "sites_per_thread 1|2|4; or, with block 64 and one site per thread, pin_mode 9|10, xcd 0|8 or a tiled "
+                  "schedule, and pin_mode 1..4, xcd 100 + a tiled schedule");
     g_forced.store(pin_mode | block << 4 | xcd << 16 | sites_per_thread << 24);
     return CLG_OK;
 }

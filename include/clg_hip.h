@@ -496,15 +496,19 @@ int clg_autotune_enable(int mode);
  * parities block by block) | 1 (XCD slabs, parities one after the other) | 10*TY + m with TY in 2, 4, 8
  * (staged modes only: the (x,y) planes cut into 8 tiles, 8/TY along x and TY along y, XCD k sweeping
  * tile k x-major (m = 0) or y-major (m = 1)), sites_per_thread 1|2|4 (0 = 1: consecutive blocks of
- * sites per workgroup); pin_mode 0 clears */
+ * sites per workgroup); pin_mode 0 clears.
+ * With block 64 and one site per thread also the launches in 64-site blocks, for any lattice: pin_mode 9
+ * (direction-split: eight waves share 64 sites, one hop direction each) | 10 (the same with
+ * non-temporal link loads) with xcd 0 | 8 | 10*TY + m, and pin_mode 1..4 with xcd 100 + 10*TY + m */
 int clg_autotune_force(int pin_mode, int block, int xcd, int sites_per_thread);
 /* Tuned configurations persist across processes when the environment variable CLG_TUNE_CACHE names a
  * file: every tuned key is appended as one line "<device arch> <tuner> <key> : <configuration>", and
  * the tuners take the lines of the current device architecture from the file before timing a key
  * (again after clg_autotune_reset).  Lines that do not parse, or configurations no launch accepts,
  * are skipped. */
-/* The staggered D tunes its own launch (block 64|128|256, hardware or XCD-slab order, pinning);
- * the environment variable CLG_TUNE_FORCE_KS="block,xcd,pin" (xcd 0|8, pin 0|2) fixes it. */
+/* The staggered D tunes its own launch; the environment variable CLG_TUNE_FORCE_KS="block,xcd,pin"
+ * fixes it: block 64|128|256, xcd 0|8, pin 0|2 (one site per thread), or block 64, xcd 0 | 8 |
+ * 10*TY + m, pin 9 (direction-split). */
 /* forget every tuned shape (the next call of each shape tunes again) */
 int clg_autotune_reset(void);
 /* number of tuned shapes, and a one-line description of entry `index` */
