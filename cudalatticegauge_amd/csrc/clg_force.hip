@@ -104,21 +104,33 @@ __global__ __launch_bounds__(256) void k_wilson_force(Geo g, const char* X, cons
 }
 
 // staggered force kernel over npole (phi_i, d_i) pairs with numerators a_i.  The link does not depend on the
-// pole, so the poles' outer products are summed first,
-//   sum_i a_i [ (U phi_i(x+mu)) d_i(x)^dagger + phi_i(x) (U d_i(x+mu))^dagger ] = U M1 + M2 U^dagger,
-// and U and Ta are applied once: 84 instead of 210 FP64 operations per pole and link.  Bound by the loads in
-// flight (172 VGPRs, two waves per SIMD; at most 168 spills and is no faster) and by L2: the site's own
-// vectors are read once per workgroup, two poles a round, through LDS (straight from L1/L2 by all four
-// waves: 113 us), the next round's in flight during this one.  Measured: 24^3x8, 12 poles 143 -> 83 us;
-// 12x10x14x16, 3 poles 31 -> 14; 19x21x15x18, 1 pole 54 -> 42 (one thread per site, the four directions and
-// the whole expression per pole in turn before).
+// pole, and Ta[X^dagger] = -Ta[X], so the poles are summed first,
+//   sum_i a_i Ta[ (U phi_i(x+mu)) d_i(x)^dagger + phi_i(x) (U d_i(x+mu))^dagger ] = Ta[ U M ],
+//   M = sum_i a_i ( phi_i(x+mu) d_i(x)^dagger - d_i(x+mu) phi_i(x)^dagger ),
+// and U and Ta are applied once: 144 instead of 210 FP64 operations per pole and link, half of them to keep what
+// the sum over the poles rounds off, without which the error grows with their number.  Relative error (2-norm,
+// against long double) at 1 / 5 / 12 / 32 poles of equal size: 1.4 / 1.4 / 1.4 / 1.4e-16, of one direction and sizes
+// over two decades 1.4 / 1.3 / 1.2 / 1.2e-16; the whole expression per pole in turn 1.3 / 1.5 / 1.6 / 2.0 and
+// 1.3 / 1.2 / 1.4 / 2.0e-16, numerators on the vectors and plain sums of both outer products 1.5 / 1.6 / 1.9 / 2.4
+// and 1.5 / 1.8 / 2.2 / 3.1e-16.
+// Bound by the loads in flight (184 VGPRs, two waves per SIMD) and by L2: the site's own vectors are read once
+// per workgroup, two poles a round, through LDS (straight from L1/L2 by all four waves a third slower), the next
+// round's in flight during this one.  Measured, us a launch among others: 24^3x8, 12 poles 132 -> 70; 12x10x14x16,
+// 3 poles 29 -> 12; 19x21x15x18, 1 pole 43 -> 39 (one thread per site, the four directions and the whole expression
+// per pole in turn before); plain sums take 69, 12 and 39.
+// m += a t; lost takes what the sum rounds off (exact for |m| >= |a t|)
+__device__ __forceinline__ void add_kept(double& m, double& lost, double a, double t) {
+    const double y = fma(a, t, m);
+    lost += fma(a, t, m - y);
+    m = y;
+}
 struct PolePtrs {
     const char* phi[32];
     const char* d[32];
     double a[32];
 };
 __global__ __launch_bounds__(256) void k_ks_force(Geo g, PolePtrs pp, int npole, const char* U, char* F, int tile_y) {
-    // two poles a round: own vectors [buffer][pole, phi or d][colour][site], already times a_i
+    // two poles a round: own vectors [buffer][pole, phi or d][colour][site]
     __shared__ double2 own[2][4][3][64];
     const int mu = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
     const int Vh = g.Vh;
@@ -139,16 +151,14 @@ __global__ __launch_bounds__(256) void k_ks_force(Geo g, PolePtrs pp, int npole,
     }
     const unsigned el = (unsigned)((p * 4 + mu) * 9 * Vh + h);
     const unsigned en = (unsigned)(n.p * 3 * Vh + n.h), ex = (unsigned)(p * 3 * Vh + h);
-    cx m1[9], m2[9], mine[3] = {};
+    cx m[9], lost[9], mine[3] = {};  // M, and what rounding dropped from its sum over the poles
 #pragma unroll
-    for (int k = 0; k < 9; ++k) m1[k] = m2[k] = cx{0.0, 0.0};
+    for (int k = 0; k < 9; ++k) m[k] = lost[k] = cx{0.0, 0.0};
     // wave w brings vector w & 1 of pole r + w / 2
     auto fetch = [&](int r) {
         const int rr = r + (mu >> 1);
         if (rr >= npole) return;
         KSIO<CLG_F64>::load((mu & 1) ? pp.d[rr] : pp.phi[rr], nullptr, Vh, ex, 0u, mine);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) mine[c] = cscale(mine[c], pp.a[rr]);
     };
     fetch(0);
     for (int r = 0, buf = 0; r < npole; r += 2, buf ^= 1) {
@@ -166,28 +176,30 @@ __global__ __launch_bounds__(256) void k_ks_force(Geo g, PolePtrs pp, int npole,
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             if (r + i < npole) {
-                cx phix[3], dx[3];
+                const double ai = pp.a[r + i];
+                cx dx[3], nphix[3];
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
                     const double2 v = own[buf][2 * i][c][lane], w = own[buf][2 * i + 1][c][lane];
-                    phix[c] = cx{v.x, v.y};
+                    nphix[c] = cx{-v.x, -v.y};
                     dx[c] = cx{w.x, w.y};
                 }
-                outer_add(phin[i], dx, m1);
-                outer_add(phix, dn[i], m2);
+#pragma unroll
+                for (int k = 0; k < 9; ++k) {
+                    cx t = cmulc(dx[k % 3], phin[i][k / 3]);
+                    cfmac(t, nphix[k % 3], dn[i][k / 3]);
+                    add_kept(m[k].x, lost[k].x, ai, t.x);
+                    add_kept(m[k].y, lost[k].y, ai, t.y);
+                }
             }
         }
     }
     if (!valid) return;
     cx u[9], f[9];
     LinkIO<CLG_F64, 18>::load<true>(U, Vh, el, u);
-    su3_mm(u, m1, f);
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-#pragma unroll
-            for (int k = 0; k < 3; ++k) cfmac(f[3 * i + j], u[3 * j + k], m2[3 * i + k]);  // += M2 U^dagger
+    for (int k = 0; k < 9; ++k) m[k] = cadd(m[k], lost[k]);
+    su3_mm(u, m, f);
     su3_ta(f);
     add_link(F, Vh, el, f, ((sum & 1) != 0) == (n.sign < 0) ? -1.0 : 1.0);  // F -= eta sign f
 }
