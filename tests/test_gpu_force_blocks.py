@@ -1,5 +1,5 @@
-"""Fermion force kernels in 64-site blocks: lattices whose planes leave partly idle blocks or fill them exactly,
-odd extents, and pole counts at the edges of the two-pole rounds."""
+"""Fermion force kernels in 64-site blocks, in both work orders: XCD slabs, and the tiled order over (x, y) planes
+that lattices take where it leaves at most one lane in eight idle; pole counts at the edges of the two-pole rounds."""
 import numpy as np
 import pytest
 
@@ -8,7 +8,22 @@ import orc
 
 pytestmark = pytest.mark.gpu
 
-LATTICES = [(5, 3, 4, 4), (4, 6, 10, 14), (3, 9, 8, 16)]
+# slabs: small planes, planes of 70 sites of a parity, odd extents; then tiles: eight full ones, one empty, of one
+# and two rows, and planes of 63 and 60 sites, whose blocks are not full
+SLABS = [(5, 3, 4, 4), (4, 6, 10, 14), (3, 9, 8, 16)]
+TILES = [(2, 8, 8, 16), (2, 7, 8, 16), (3, 15, 8, 16), (3, 8, 9, 14), (2, 16, 10, 12)]
+LATTICES = SLABS + TILES
+
+
+def busy(dims):
+    """share of the lanes that the tiled order (eight tiles along y, planes in blocks of 64 sites) keeps busy"""
+    plane = dims[2] * dims[3] // 2
+    return dims[0] * dims[1] * plane / (8 * dims[0] * -(-dims[1] // 8) * -(-plane // 64) * 64)
+
+
+@pytest.mark.parametrize("dims", LATTICES)
+def test_orders(dims):
+    assert (busy(dims) >= 7 / 8) == (dims in TILES)
 
 
 def put(ctx, kind, dims, data):

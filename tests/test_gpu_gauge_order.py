@@ -1,5 +1,5 @@
-"""Gauge force and plaquette energy in 64-site blocks, on lattices whose planes leave partly idle blocks (slab
-order), fill them exactly (tiled order), or whose extents are odd, 2 or 1 tile short."""
+"""Gauge force and plaquette energy in 64-site blocks, in both work orders: XCD slabs, and the tiled order over
+(x, y) planes that lattices take where it leaves at most one lane in eight idle."""
 import numpy as np
 import pytest
 
@@ -9,8 +9,21 @@ import orc
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("dims", [(5, 3, 4, 4), (4, 6, 10, 14), (3, 9, 8, 16), (2, 2, 16, 8), (2, 11, 8, 16)])
+# small planes, planes of 70 sites of a parity, odd extents, tiles far from full
+SLABS = [(5, 3, 4, 4), (4, 6, 10, 14), (3, 9, 8, 16), (2, 2, 16, 8), (2, 11, 8, 16)]
+# eight full tiles; one tile empty; tiles of one and two rows; planes of 63 and 60 sites, whose blocks are not full
+TILES = [(2, 8, 8, 16), (2, 7, 8, 16), (3, 15, 8, 16), (3, 8, 9, 14), (2, 16, 10, 12)]
+
+
+def busy(dims):
+    """share of the lanes that the tiled order (eight tiles along y, planes in blocks of 64 sites) keeps busy"""
+    plane = dims[2] * dims[3] // 2
+    return dims[0] * dims[1] * plane / (8 * dims[0] * -(-dims[1] // 8) * -(-plane // 64) * 64)
+
+
+@pytest.mark.parametrize("dims", SLABS + TILES)
 def test_force_and_energy(dims):
+    assert (busy(dims) >= 7 / 8) == (dims in TILES)
     U = orc.gauge_random(dims, 0.4, 1)
     rng = np.random.default_rng(2)
     F0 = rng.standard_normal(U.size)
