@@ -11,8 +11,8 @@
 //     workgroup size and the work order per batch shape).  Segments after one another read the
 //     links from the last-level cache once each; in turns (BSeg::grp, with XCD slabs) the segments
 //     of one gauge field meet in one XCD's L2.  Measured, 12 right-hand sides at 16^3x32 and three
-//     small lattices: FP64 half hop 217 -> 164 us, with the x term 241 -> 183, both parities
-//     433 -> 352; FP16 vectors 50.5 -> 44.8;
+//     small lattices, back to back: FP64 half hop 217 -> 164 us, with the x term 241 -> 183, both
+//     parities 433 -> 352; FP16 vectors 50.5 -> 44.8 (48 to 51 in a solve, between other kernels);
 //   * the Krylov BLAS runs on a 2-D grid (blocks x systems) with per-system reductions;
 //   * each system keeps its own Krylov space and GMRES(m) recurrences, so every solution is the
 //     one the single-system solver produces (same algorithm, same stopping rule per system).
@@ -716,15 +716,14 @@ __global__ void k_bzero(const BTab* T, Act act, int ysel) {
 }
 
 // ---- per-system small kernels (one workgroup per system): Hessenberg update and least squares
-// Per-system workspace: H (2 ld m), c2 (2m), g (2(m+1)), y (2m), sc (16) doubles, then an int area.
+// Per-system workspace: H (2 ld m), c2 (2m), y (2m), sc (16) doubles, then the Gram-Schmidt block (40).
 struct WsLayout {
     int m, ld;
-    size_t offH, offC, offG, offY, offS, offGS, stride;
+    size_t offH, offC, offY, offS, offGS, stride;
     WsLayout(int m_) : m(m_), ld(m_ + 1) {
         offH = 0;
         offC = offH + 2 * (size_t)ld * m;
-        offG = offC + 2 * (size_t)m;
-        offY = offG + 2 * (size_t)(m + 1);
+        offY = offC + 2 * (size_t)m;
         offS = offY + 2 * (size_t)m;
         offGS = offS + 16;
         stride = offGS + 40;
@@ -888,9 +887,9 @@ __global__ __launch_bounds__(kRedBlock) void k_bh_multidot(const BTab* T, Act ac
 // w' = w - sum_k h_k V_k, stored to vector osel (w itself or the next basis vector), with the
 // partials of V_k^H w' and |w'|^2; h at ws[s*stride + offh].  Per system, when |w|^2 - |h|^2 keeps half
 // of |w|^2 (no second pass needed), w'/|w'| is stored and no partials are taken; the system's workgroup 0
-// records the choice in its Gram-Schmidt block (gs[1] |w'|^2, gs[2] 1/|w'|, gs[3] 2 for the fast form, else 0).  last: the cycle's last step, whose
-// vector nothing reads: the fast form stores none (15 systems, 12 of them 16^3x32, 12 vectors: a pass of 131 us
-// less a cycle, batched solve 13.70 -> 13.38 ms).
+// records the choice in its Gram-Schmidt block (gs[1] |w'|^2, gs[2] 1/|w'|, gs[3] 2 for the fast form, else
+// 0).  last: the cycle's last step, whose vector nothing reads: the fast form stores none (15 systems, 12 of
+// them 16^3x32, 12 vectors: a pass of 131 us less a cycle, batched solve 13.70 -> 13.38 ms).
 template <int K>
 __global__ __launch_bounds__(kRedBlock) void k_bh_gs_project(const BTab* T, Act act, int wsel, int osel, double* ws,
                                                               int stride, int offh, double* partial, int offgs,

@@ -318,8 +318,8 @@ __global__ __launch_bounds__(kFinBlock) void k_red_finish_ch(const double* __res
 // Second stage of the BLAS reductions (one workgroup): total_r = sum over nblk partials of
 // partial[b * NR + r] in a fixed order; totals r < nout go to out[r], the one after them to
 // out2[0] (when given).  flag (nullable): *flag = (total_0 < eta * ref[0]).  cond (nullable): skip
-// when *cond == 0, as the first stage did.  Every load of a thread is independent (block-major
-// sweep with NR accumulators), so they all stay in flight.
+// when *cond == 0, as the first stage did.  partial_totals does the sums: a thread takes one value of every
+// G-th block, so its loads are independent and neighbouring threads read neighbouring values.
 __global__ __launch_bounds__(kFinBlock) void k_red_finish(const double* __restrict__ partial, int nblk, int nr, double* out,
                                                           int nout, double* out2, const int* cond, const double* ref,
                                                           double eta, int* flag) {
@@ -398,8 +398,8 @@ __device__ __forceinline__ void gs_slow_column(const double* tot, double* hcol, 
         double c2 = 0;
         for (int k = 0; k < 2 * K; ++k) c2 += tot[k] * tot[k];
         double f2 = flag ? w2 - c2 : w2;
-        // w lies in the span (its norm is below the rounding of the subtraction): an invariant subspace.  The next
-        // vector is zero, not the noise divided by a tiny norm; NaN stays NaN
+        // nothing is left of w (|w''|^2 comes out below 1e-300 or negative): an invariant subspace, and the next
+        // vector is zero.  Positive noise of the subtraction is normalised like any other vector; NaN stays NaN
         const bool none = f2 <= 1e-300;
         const double f = none ? 0.0 : sqrt(f2);
         hcol[2 * (j + 1)] = shifted ? -f : f;
@@ -635,8 +635,9 @@ __global__ __launch_bounds__(kFinBlock) void k_gs_fast_last(const double* __rest
     (void)gs_fast_scalars<K>(tot, tot[2 * K], hcol, j, sc);
 }
 
-// workgroups of a reduction: four packets a lane, but one a lane while that gives at most kMergeGrid workgroups (a
-// small vector's pass is a chain of latencies: 12-vector multi-dot at 8^4 7.9 -> 4.4 us)
+// workgroups of a reduction: one packet a lane up to kMergeGrid workgroups (65536 packets), then kMergeGrid of them
+// with up to four a lane (262144), then four a lane up to the cap.  (A small vector's pass is a chain of latencies:
+// 12-vector multi-dot at 8^4 7.9 -> 4.4 us with one a lane instead of four.)
 unsigned red_grid(clg_context ctx, long n) {
     const long one = (n + kRedBlock - 1) / kRedBlock, four = (one + 3) / 4;
     const long cap = std::min<long>(kMaxRedGrid, (long)ctx->num_cu * 4);
@@ -798,7 +799,6 @@ int blas_conj(clg_context ctx, clg_field_s* dst, const clg_field_s* src) {
     return CLG_OK;
 }
 
-// second stage of a reduction whose first stage wrote nblk * nr partials to ctx->red_partial
 // second stage of a reduction whose first stage wrote nblk x nr partials to `partial`
 static int red_finish_at(clg_context ctx, const double* partial, unsigned nblk, int nr, double* out, int nout,
                          double* out2, const int* cond, const double* ref, double eta, int* flag) {

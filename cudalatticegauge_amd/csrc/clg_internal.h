@@ -288,8 +288,8 @@ inline bool tile64_fits(const Geo& g, int TY) {
 
 // work order of the site kernels in 64-site blocks: the tiled plane order where it keeps the lanes busy
 // (neighbour planes then meet in one XCD's L2), else XCD slabs.  Gauge force at 32^3x16: eight tiles along y
-// 322 us, 2 x 4 tiles 341, 4 x 2 tiles 346, slabs 344; at 21x19x25x18, where a plane fills 4 of 3.5 blocks,
-// all within 1 %.
+// 322 us, 2 x 4 tiles 341, 4 x 2 tiles 346, slabs 344; at 21x19x25x18, where a plane of 225 sites fills 3.5 of 4
+// blocks and the tiles at most 0.80 of the lanes, all within 1 %.
 struct SiteOrder {
     int tile_y;  // 0: slabs
     unsigned grid;
@@ -1115,7 +1115,7 @@ __device__ void block_partial(double (&v)[NR], double* partial) {
 
 // Totals tot[0..nr) (LDS) of nblk x nr row-major partials by one workgroup of BLOCK threads, in a fixed order:
 // thread (q, r) sums value r of blocks q, q + G, ..., neighbouring threads reading neighbouring values, then
-// 8 to 32 strands and one fold the G rows.  nr <= kFinMax.  Measured for 25 values of 24 blocks: the finish 5.5 ->
+// up to 32 strands (never more than G) and one fold the G rows.  nr <= kFinMax.  Measured for 25 values of 24 blocks: the finish 5.5 ->
 // 3.8 us (a thread per block with nr strided accumulators and nr wave butterflies before).
 constexpr int kFinBlock = 1024, kFinMax = 33;
 template <int BLOCK>
@@ -1148,9 +1148,8 @@ __device__ __forceinline__ void partial_totals(const double* __restrict__ partia
 // rotations and back substitution as RotateH / SolveY (CSolverGMRES.cpp:262-358), FP64.  H is column-major with
 // leading dimension ld; sm holds m * ld complex numbers of LDS.  Lane j carries column j: a rotation is one
 // broadcast and four products a lane, and the back substitution eliminates column by column.  A column of
-// zeros (the vectors after an invariant subspace) gets y = 0.  dev[0] = |g_m|^2,
-// dev[1] = |g_m|.  Measured for m = 12: 7.7 us (one thread on
-// global memory: 28).
+// zeros (the vectors after an invariant subspace) gets y = 0.  dev[0] = |g_m|^2, dev[1] = |g_m|.  Measured for
+// m = 12: 7.7 us (one thread on global memory: 28).
 __device__ __forceinline__ cd lane_bcast(cd a, int src) { return cd{__shfl(a.x, src, 64), __shfl(a.y, src, 64)}; }
 // With *bad set (a refused fast Gram-Schmidt step in the cycle) y is zero; dev[2] passes it on.
 __device__ __forceinline__ void gmres_lsq_wave(const double* __restrict__ H, int ld, int m, double beta2, double* y,

@@ -394,7 +394,8 @@ __global__ __launch_bounds__(kBcgBlock) void k_bcg_norms(long n, int ns, BcgShif
 
 enum { FIN_INIT = 0, FIN_CHECK = 1 };
 
-// totals of the G workgroups' partials, then the initial scalars or the check's.  One workgroup: thread 0 the global scalars, thread k < ns shift k.
+// totals of the G workgroups' partials, then the initial scalars or the check's.  One workgroup: thread 0 the global
+// scalars, thread k < ns shift k.
 template <int NR, int STAGE>
 __global__ __launch_bounds__(kFinBlock) void k_bcg_fin(const double* __restrict__ part, int G, double* st, int ns,
                                                        double bound) {

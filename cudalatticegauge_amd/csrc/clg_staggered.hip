@@ -138,7 +138,7 @@ __global__ __launch_bounds__(256) void k_ks(KSArgs a) {
 // c < 3 sums colour c, adds the mass or x term and stores.  Eight times the waves for a small lattice, and
 // both users of a link in one L2 more often on a large one.  Measured (us, one site per thread -> split):
 // FP64 D 21x19x25x18 27.1 -> 24.7, 24^3x24 47.9 -> 36.2 (tiled order), 24^3x48 108 -> 91, FP32 24^3x16
-// 17.4 -> 15.3; FP16 storage loses from 12^3x24 on (5.0 against 5.4).  The tuner times both.
+// 17.4 -> 15.3; FP16 storage loses from 16^4 on (4.6 against 5.1).  The tuner times both.
 constexpr int kSplitSites = 64;
 
 template <int MU, bool FWD, typename R, class SIO, class LIO>
@@ -317,7 +317,8 @@ bool ks_valid(const KSCfg& c) {
 
 // Untuned launches (tuning off, small lattices, graph capture) take the direction split up to this many
 // sites: measured, it is level with one site per thread or ahead of it for FP64 and FP32 vectors (FP64 D at
-// 24^3x16 29.2 against 32.5 us) and behind in FP16 from 12^3x24 on (5.4 against 5.0 us).
+// 24^3x16 28.1 against 32.1 us); in FP16 it is ahead at 12^4 (3.7 against 4.6), level at 12^3x24 (4.5) and
+// behind from 16^4 on (5.1 against 4.6).
 inline long split_default_max(int prec) { return prec == CLG_F16 ? 32768 : 262144; }
 
 int ks_launch(const KSArgs& a, int prec, int gprec, bool r12, hipStream_t st) {

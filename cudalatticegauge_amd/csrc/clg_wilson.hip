@@ -169,9 +169,10 @@ __global__ __launch_bounds__(256) void k_wilson_hop(HopArgs a) {
 // the XCD's L2: with the tiled order (tile64_site) it also leads on lattices that fill the chip.  Measured
 // (us, one site per thread -> split): FP64 D 8^4 7.6 -> 5.0, 24^3x24 101 -> 66, 32^4 311 -> 256; FP32 D
 // 24^3x48 95 -> 67; half hops FP64 16^4 11.7 -> 9.7, 32^4 154 -> 143 (non-temporal links), FP32 16^4 7.9 ->
-// 5.9, 24^3x48 49 -> 38.  It loses where one thread per site is already bound by memory with little state:
-// FP16 storage from 16^4 on (32^4 half hop 34 against 41), and FP64 D at 32^3x16 (122 against 125, staged).
-// The tuner times both.
+// 5.9, 24^3x48 49 -> 38; FP16 storage, D 12^4 7.3 -> 4.5, half hops 16^4 6.7 -> 4.7, 24^3x16 11.3 -> 10.7.  It
+// loses where one thread per site is already bound by memory with little state: FP16 storage on larger lattices
+// (half hop 32^3x16 18.6 against 22.0, 32^4 33 against 40; D from 16^3x32 on, 11.5 against 11.8), and is level
+// with the staged launches for FP64 D at 32^3x16 (122 against 124).  The tuner times both.
 constexpr int kSplitSites = 64;
 
 // U h (forward) or U^dagger h (backward) of the neighbour in direction MU
@@ -488,8 +489,9 @@ bool forced_cfg(HopCfg& c) {
 
 // Untuned launches (tuning off, small lattices, graph capture) take the direction split up to this many
 // sites: measured, it is ahead of one site per thread for FP64 and FP32 spinors in the XCD-slab order up to
-// here (FP64 D at 24^3x16 48.6 against 61.2 us, FP32 26.7 against 27.7) and behind in FP16 from 16^4 on
-// (8.4 against 8.1 us).
+// here (FP64 D at 24^3x16 48.6 against 61.2 us, FP32 26.7 against 27.7).  In FP16 it is well ahead up to
+// 12^3x24 (D 5.9 against 7.9 us), less so at 16^4 (7.0 against 8.1), level at 16^3x32 (11.9) and behind at
+// 32^3x16 (half hop 21.8 against 18.8, D 40 against 35): the line lies where the gain is still large.
 inline long split_default_max(int prec) { return prec == CLG_F16 ? 32768 : 262144; }
 
 int launch_hop(const HopArgs& a, int prec, int gprec, int recon, bool dag, bool hasx, hipStream_t st) {
@@ -564,8 +566,12 @@ int launch_hop(const HopArgs& a, int prec, int gprec, int recon, bool dag, bool 
                             if (m == 0 && TY >= 4) all.push_back(HopCfg{pm, sb, 10 * TY + m, 1, 1});
                         }
         }
-        // Links that fit the 32 MB of L2 are read from there by the next hops: no non-temporal loads of them.  The
-        // tuner's own launches cannot show it (FP32 half hops at 16^4 in a solve: 6.6 us, non-temporal 9.4).
+        // Links that fit the 32 MB of L2 are read from there by the next hops: no non-temporal loads of them.  Best
+        // cached against best non-temporal launch, us, each repeated: FP64 D 12^3x16 (15 MB) 6.7 / 8.1, 16^3x12
+        // (27 MB) 11.5 / 13.7, half hop 7.4 / 8.6; FP32 D 16^4 (18 MB) 8.6 / 11.0, 16^3x24 (27 MB) 12.8 / 16.1, half
+        // hop 7.1 / 8.0; FP16 D 24^3x16 (20 MB) 18.1 / 19.7; level where everything is small (8^4).  Between the
+        // other kernels of a solve the gap is wider (FP32 half hops at 16^4 6.6 / 9.4) than a candidate's few
+        // launches show.
         if (8L * a.g.Vh * (recon == 12 ? 12 : 18) * (gprec == CLG_F64 ? 8 : gprec == CLG_F32 ? 4 : 2) <= (32L << 20))
             all.erase(std::remove_if(all.begin(), all.end(),
                                      [](const HopCfg& c) {

@@ -1,6 +1,7 @@
-"""Batched hops whose segments of one gauge field take turns workgroup by workgroup: every system as a launch of its own
-gives it (with one right-hand side per thread bit for bit: a site's sum does not depend on the order of the sites), for one to several segments per gauge
-field, gauge fields in mixed order, lattices that end in part of a workgroup, and different coefficients."""
+"""Batched hops whose segments of one gauge field take turns workgroup by workgroup: every system as a launch of its
+own gives it (with one right-hand side per thread bit for bit: a site's sum does not depend on the order of the
+sites), for one to several segments per gauge field, gauge fields in mixed order, lattices that end in part of a
+workgroup, and different coefficients."""
 import numpy as np
 import pytest
 
