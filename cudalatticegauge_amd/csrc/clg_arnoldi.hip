@@ -41,8 +41,8 @@ template <int P> struct ArnPtrs {
     const typename Pk<P>::T* p[kArnMaxV];
 };
 
-// scratch layout (doubles): [0] |w|^2, [1] |w''|^2, [2] 1/|w''| (0 when w lies in the span), [3] the flag (as an int), [4, 4+128)
-// c2, [132, 132+128) h
+// scratch layout (doubles): [0] |w|^2, [1] |w''|^2, [2] 1/|w''| (0 when w lies in the span), [3] the flag (as an
+// int), [4, 4+128) c2, [132, 132+128) h
 constexpr int kScFlag = 3, kScC2 = 4, kScH = 4 + 2 * kArnMaxV;
 
 __device__ __forceinline__ int arn_flag(const double* sc) { return *reinterpret_cast<const int*>(sc + kScFlag); }

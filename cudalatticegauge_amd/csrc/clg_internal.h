@@ -1115,8 +1115,8 @@ __device__ void block_partial(double (&v)[NR], double* partial) {
 
 // Totals tot[0..nr) (LDS) of nblk x nr row-major partials by one workgroup of BLOCK threads, in a fixed order:
 // thread (q, r) sums value r of blocks q, q + G, ..., neighbouring threads reading neighbouring values, then
-// up to 32 strands (never more than G) and one fold the G rows.  nr <= kFinMax.  Measured for 25 values of 24 blocks: the finish 5.5 ->
-// 3.8 us (a thread per block with nr strided accumulators and nr wave butterflies before).
+// up to 32 strands (never more than G) and one fold the G rows.  nr <= kFinMax.  Measured for 25 values of 24
+// blocks: the finish 5.5 -> 3.8 us (a thread per block with nr strided accumulators and nr wave butterflies before).
 constexpr int kFinBlock = 1024, kFinMax = 33;
 template <int BLOCK>
 __device__ __forceinline__ void partial_totals(const double* __restrict__ partial, int nblk, int nr, double* tot) {

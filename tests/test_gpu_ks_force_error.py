@@ -39,7 +39,8 @@ def test_error(poles, alike):
     a = np.linspace(0.1, 1.0, poles)
     if alike:  # solutions of one source at growing shifts
         size = 1 / (0.05 + np.logspace(-4, 1, poles))
-        phis, ds = ([s * (orc.ks_gaussian(DIMS, 98 + k) + 0.3 * v) for s, v in zip(size, vs)] for k, vs in enumerate((phis, ds)))
+        phis, ds = ([s * (orc.ks_gaussian(DIMS, 98 + k) + 0.3 * v) for s, v in zip(size, vs)]
+                    for k, vs in enumerate((phis, ds)))
         a = 0.01 * np.logspace(0, 2, poles)
     with clg.Context(0) as ctx:
         def put(kind, data):
